@@ -16,7 +16,8 @@
 //                       probability-weighted value sums.  The last workgroup
 //                       of a (sequence, head) to arrive merges the chunks
 //                       (rescaled by exp(m_chunk - m)) and writes bf16
-//                       (model.py:61-122).
+//                       (model.py:61-122).  Batch 1 and up to 16 chunks;
+//                       larger calls take qwen2_decode_split.hip.
 //   prefill_rope_kernel, prefill_attention_kernel
 //                       a prompt: rotary of every position (queries to a
 //                       workspace, keys and values into the caches), then
@@ -49,10 +50,8 @@ constexpr int kPartFloats = 2 * kMaxGroup + kMaxGroup * kHeadDim;  // m[8], l[8]
 static_assert(kPartFloats == kAttnPartFloats && kChunk == kAttnChunk && kMaxGroup == kAttnMaxGroup &&
                   kHeadDim == kAttnHeadDim,
               "the partial-result layout the attention-merge GEMV reads");
-constexpr int kMergeBatch = 16;   // chunks whose partial sums one merge pass loads together
-// The merge keeps per-chunk statistics in the staging rows' LDS.
-constexpr int kMaxChunks = (kChunk * kRowStride * 2) / (2 * kMaxGroup * 4);
-constexpr int kMaxLength = kMaxChunks * kChunk;
+constexpr int kMergeChunks = kAttnMergeMaxChunks;  // chunks one workgroup merges (more: qwen2_decode_split.hip)
+constexpr int kMaxLength = 17408;
 
 
 // Thread t owns the 8-element pieces 8 t + 2048 i (i < kNormIters).  Every
@@ -469,57 +468,46 @@ __global__ __launch_bounds__(kAttnThreads) void attention_kernel(AttnArgs a) {
     // After the acquire, plain loads see every other workgroup's partials.
     // The merge issues them all at once: the statistics first (their loads
     // return first), then per thread t < group * 32 the weighted sums of head
-    // t / 32, dimensions 4 (t % 32) .. + 3, of up to kMergeBatch chunks as
+    // t / 32, dimensions 4 (t % 32) .. + 3, of the up to 16 chunks as
     // 16-byte loads.  Loads of chunks past `used` (or threads past the
     // group's heads) re-read a valid partial; their scale is zero (or their
     // result is not stored), so the accumulation needs no branches.
     const int used = pos / kChunk + 1;  // chunks that hold positions 0..pos (all wrote partials)
     const float* base = a.partials + (int64_t)slot * a.chunks * kPartFloats;
     float* stats = (float*)&ks[0][0];    // [used][2 * kMaxGroup]: m, l per head
-    float* scale_c = (float*)&vt[0][0];  // [kMaxChunks][kMaxGroup]: exp(m_c - m) / l, zero past `used`
-    for (int e = tid; e < used * 2 * kMaxGroup; e += kAttnThreads)
-        stats[e] = base[(e / (2 * kMaxGroup)) * kPartFloats + e % (2 * kMaxGroup)];
+    float* scale_c = (float*)&vt[0][0];  // [kMergeChunks][kMaxGroup]: exp(m_c - m) / l, zero past `used`
+    static_assert(kMergeChunks * 2 * kMaxGroup == kAttnThreads, "one statistic per thread");
+    if (tid < used * 2 * kMaxGroup) stats[tid] = base[(tid / (2 * kMaxGroup)) * kPartFloats + tid % (2 * kMaxGroup)];
     const int f = min(tid, group * (kHeadDim / 4) - 1);
     const int gh = f / (kHeadDim / 4);     // head within the group
     const int d4 = 4 * (f % (kHeadDim / 4));  // first of its four dimensions
-    float4v v[kMergeBatch];
-    auto load_batch = [&](int c0) {
+    float4v v[kMergeChunks];
 #pragma unroll
-        for (int u = 0; u < kMergeBatch; ++u)
-            v[u] = *(const float4v*)(base + min(c0 + u, used - 1) * kPartFloats + 2 * kMaxGroup + gh * kHeadDim + d4);
-    };
-    load_batch(0);
+    for (int u = 0; u < kMergeChunks; ++u)
+        v[u] = *(const float4v*)(base + min(u, used - 1) * kPartFloats + 2 * kMaxGroup + gh * kHeadDim + d4);
     __syncthreads();
-    // per head g (wave w takes heads w, w + 4): lanes walk the chunks; the
+    // per head g (wave w takes heads w, w + 4): lane c holds chunk c; the
     // head's maximum and rescaled sum are wave reductions.  Heads past
     // `group` get zero scales.
     for (int g = wave; g < kMaxGroup; g += kAttnThreads / 64) {
         if (g >= group) {
-            for (int c = lane; c < kMaxChunks; c += 64) scale_c[c * kMaxGroup + g] = 0.0f;
+            if (lane < kMergeChunks) scale_c[lane * kMaxGroup + g] = 0.0f;
             continue;
         }
-        float m = -INFINITY;
-        for (int c = lane; c < used; c += 64) m = fmaxf(m, stats[c * 2 * kMaxGroup + g]);
-        m = wave_max(m);
-        float l = 0.0f;
-        for (int c = lane; c < used; c += 64)
-            l = fmaf(stats[c * 2 * kMaxGroup + kMaxGroup + g], expf(stats[c * 2 * kMaxGroup + g] - m), l);
-        l = wave_sum(l);
-        for (int c = lane; c < kMaxChunks; c += 64)
-            scale_c[c * kMaxGroup + g] = c < used ? expf(stats[c * 2 * kMaxGroup + g] - m) / l : 0.0f;
+        const float mc = lane < used ? stats[lane * 2 * kMaxGroup + g] : -INFINITY;
+        const float m = wave_max(mc);
+        const float l =
+            wave_sum(lane < used ? fmaf(stats[lane * 2 * kMaxGroup + kMaxGroup + g], expf(mc - m), 0.0f) : 0.0f);
+        if (lane < kMergeChunks) scale_c[lane * kMaxGroup + g] = lane < used ? expf(mc - m) / l : 0.0f;
     }
     __syncthreads();
     W4G64_STAMP(6);
     float4v o = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int c0 = 0; c0 < used; c0 += kMergeBatch) {
-        if (c0 > 0) load_batch(c0);
 #pragma unroll
-        for (int u = 0; u < kMergeBatch; ++u) {
-            float sc = scale_c[min(c0 + u, kMaxChunks - 1) * kMaxGroup + gh];
-            sc = c0 + u < used ? sc : 0.0f;
+    for (int u = 0; u < kMergeChunks; ++u) {
+        const float sc = scale_c[u * kMaxGroup + gh];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = fmaf(v[u][i], sc, o[i]);
-        }
+        for (int i = 0; i < 4; ++i) o[i] = fmaf(v[u][i], sc, o[i]);
     }
     if (tid < group * (kHeadDim / 4)) {
         const uint32_t lo = float_to_bf16_bits(o[0]) | ((uint32_t)float_to_bf16_bits(o[1]) << 16);
@@ -898,6 +886,30 @@ static int decode_attention(const void* qkv, const void* cos, const void* sin, v
     const int64_t chunks = (max_length + kChunk - 1) / kChunk;
     const int64_t blocks = batch * num_kv_heads * chunks;
     if (blocks > 0x7FFFFFFF) return set_error(W4G64_STATUS_INVALID_VALUE, "problem too large");
+    // Batch 1 with a cache of up to 1024 positions: the single kernel, whose
+    // chunks and merge are those of the o_proj linear's own merge
+    // (w4g64_linear_attention_merge), so the two forms agree bit for bit.  It
+    // is also as fast there (position 575 of 640: 7.9 us either way).  Past
+    // that the split kernel is the faster one at every size measured (2 x 640
+    // positions 8.1 -> 8.0 us, 24 x 1024 28.0 -> 11.7, 8 x 4096 51 -> 12.7):
+    // each chunk's arrival costs an agent-scope release.
+    if (!unmerged && (batch > 1 || chunks > kAttnMergeMaxChunks)) {
+        DecodeSplitArgs sp;
+        sp.qkv = (const uint16_t*)qkv;
+        sp.cos = (const uint16_t*)cos;
+        sp.sin = (const uint16_t*)sin;
+        sp.k_cache = (uint16_t*)k_cache;
+        sp.v_cache = (uint16_t*)v_cache;
+        sp.position = position;
+        sp.out = (uint16_t*)out;
+        sp.partials = (float*)((char*)workspace + attention_counter_bytes(batch, num_kv_heads));
+        sp.heads = (int)num_heads;
+        sp.kv_heads = (int)num_kv_heads;
+        sp.max_len = (int)max_length;
+        sp.splits = decode_splits(batch, num_kv_heads, max_length);
+        sp.scale2 = scale * 1.4426950408889634f;
+        return launch_status(launch_decode_split(sp, batch, (hipStream_t)stream), "decode_attention");
+    }
     AttnArgs args;
     args.qkv = (const uint16_t*)qkv;
     args.cos = (const uint16_t*)cos;

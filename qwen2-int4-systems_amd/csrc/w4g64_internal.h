@@ -137,6 +137,28 @@ constexpr int kAttnPartFloats = 2 * kAttnMaxGroup + kAttnMaxGroup * kAttnHeadDim
 inline int64_t attention_counter_bytes(int64_t batch, int64_t kv_heads) {
     return (batch * kv_heads * (int64_t)sizeof(unsigned) + 255) / 256 * 256;
 }
+// Decode attention with the context split over workgroups
+// (qwen2_decode_split.hip); partials: [batch * kv_heads][splits][kAttnPartFloats],
+// maxima in base-2 units.
+struct DecodeSplitArgs {
+    const uint16_t* qkv;
+    const uint16_t* cos;
+    const uint16_t* sin;
+    uint16_t* k_cache;
+    uint16_t* v_cache;
+    const int64_t* position;
+    uint16_t* out;
+    float* partials;
+    int heads;
+    int kv_heads;
+    int max_len;
+    int splits;
+    float scale2;  // scale * log2(e)
+};
+constexpr int kDecodeMaxSplits = 64;
+int decode_splits(int64_t batch, int64_t kv_heads, int64_t max_length);
+hipError_t launch_decode_split(const DecodeSplitArgs& args, int64_t batch, hipStream_t stream);
+
 // Chunks the attention-merge form of the pipelined GEMV takes (the cache's
 // max_length up to 1024 positions): it loads every chunk's partial result.
 constexpr int kAttnMergeMaxChunks = 16;

@@ -172,6 +172,59 @@ def test_decode_attention_matches_torch(batch, heads, kv_heads, max_length, posi
             assert cos_sim.item() >= 0.99999, (pos, cos_sim.item())
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,max_length,positions", [
+    (2, 12, 2, 64, (0, 1, 30, 31, 32, 63)),         # one split: no merge launch
+    (3, 8, 1, 129, (0, 15, 16, 127, 128)),          # two splits, the cache ends one row into a block
+    (2, 3, 3, 1000, (3, 126, 511, 512, 999)),       # one query head per key/value head, a ragged last block
+    (33, 14, 2, 300, (0, 200, 299)),                # seven per head; fewer splits than the cache has room for
+    (1, 16, 2, 17408, (31, 4095, 17407)),           # the longest cache, the most splits
+    (2, 12, 2, 640, (-5, 640, 10_000)),             # clamped to the cache
+])
+def test_decode_attention_split_over_workgroups(batch, heads, kv_heads, max_length, positions):
+    """qwen2_decode_attention past one sequence or 1024 positions (the split
+    kernel and its merge) against the same in fp64 from the rounded rotary
+    step: the fp32 result differs from it by a few fp32 ulp of the sums, so
+    the bf16 output by at most one rounding (2^-8 of the value) plus 2^-16 of
+    the largest one.  Rows past the position are NaN and must not be read into
+    the result; the workspace starts as NaN."""
+    lib = _lib.load()
+    g = _gen(batch * 100 + heads + max_length)
+    d = 128
+    rot = RotaryEmbedding(d, 1_000_000.0).cuda()
+    base = torch.randn((2, batch, kv_heads, max_length, d), generator=g, device="cuda").to(torch.bfloat16)
+    wbytes = lib.qwen2_decode_attention_workspace_bytes(batch, kv_heads, max_length)
+    counters = (batch * kv_heads * 4 + 255) // 256 * 256
+    for at in positions:
+        pos = min(max(at, 0), max_length - 1)
+        k_cache, v_cache = base.clone().unbind(0)
+        k_cache[:, :, pos:], v_cache[:, :, pos:] = float("nan"), float("nan")
+        qkv = (torch.randn((batch, (heads + 2 * kv_heads) * d), generator=g, device="cuda") * 2).to(torch.bfloat16)
+        cos, sin = rot(torch.tensor([[pos]], device="cuda").expand(batch, 1), torch.bfloat16)
+        cos, sin = cos.reshape(batch, d).contiguous(), sin.reshape(batch, d).contiguous()
+        ws = torch.full((wbytes,), 0xFF, dtype=torch.uint8, device="cuda")
+        ws[:counters] = 0
+        out = torch.empty((batch, heads * d), dtype=torch.bfloat16, device="cuda")
+        position = torch.tensor([at], dtype=torch.long, device="cuda")
+        _lib.check(lib.qwen2_decode_attention(
+            _p(qkv), _p(cos), _p(sin), _p(k_cache), _p(v_cache), _p(position), _p(out), batch, heads, kv_heads,
+            d, max_length, ctypes.c_float(d ** -0.5), _p(ws), ws.numel(), _stream()))
+        torch.cuda.synchronize()
+        q, k, v = (t.view(batch, -1, 1, d) for t in qkv.split([heads * d, kv_heads * d, kv_heads * d], dim=1))
+        c, s = cos.view(batch, 1, 1, d), sin.view(batch, 1, 1, d)
+        q, k = q * c + rotate_half(q) * s, k * c + rotate_half(k) * s
+        want_k, want_v = base.clone().unbind(0)
+        want_k[:, :, pos], want_v[:, :, pos] = k[:, :, 0], v[:, :, 0]
+        assert torch.equal(k_cache[:, :, : pos + 1], want_k[:, :, : pos + 1])
+        assert torch.equal(v_cache[:, :, : pos + 1], want_v[:, :, : pos + 1])
+        assert bool(torch.isnan(k_cache[:, :, pos + 1:]).all()) and bool(torch.isnan(v_cache[:, :, pos + 1:]).all())
+        keys, values = want_k[:, :, : pos + 1].double(), want_v[:, :, : pos + 1].double()
+        scores = (q.view(batch, kv_heads, -1, 1, d).double() * keys.unsqueeze(2)).sum(-1) * d ** -0.5
+        probs = torch.softmax(scores, dim=-1)
+        want = (probs @ values).reshape(batch, heads * d)
+        err = (out.double() - want).abs()
+        assert bool((err <= want.abs() * 2.0 ** -8 + want.abs().max() * 2.0 ** -16).all()), (at, err.max().item())
+
+
 @pytest.mark.parametrize("heads,kv_heads,max_length,positions,n,with_bias", [
     (12, 2, 640, (0, 1, 63, 64, 65, 511, 639), 1536, False),
     (12, 2, 1024, (0, 700, 1023), 1536, True),  # 16 chunks: the most the merge form takes
