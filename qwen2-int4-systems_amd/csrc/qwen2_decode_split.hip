@@ -40,8 +40,7 @@
 
 #include <type_traits>
 
-#include "w4g64_device.h"
-#include "w4g64_internal.h"
+#include "qwen2_attention.h"
 
 namespace w4g64 {
 namespace {
@@ -55,28 +54,6 @@ struct Kv {
     u32x4 k[2][4];  // key tile t, dimensions 32 sl + 8 q ..: 16-byte pieces
     u32x4 v[8];     // value of key 16 (e / 4) + 4 q + e % 4, dimensions 8 j ..
 };
-
-// Maximum / sum over the four lanes j, j + 16, j + 32, j + 48.  (The swapped
-// pair is bit cast as a whole: a bit cast of one element of the builtin's
-// integer pair compiles to element 0 with this compiler.)
-__device__ __forceinline__ float2v swap16(float v) {
-    const uint32_t a = __builtin_bit_cast(uint32_t, v);
-    return __builtin_bit_cast(float2v, __builtin_amdgcn_permlane16_swap(a, a, false, false));
-}
-__device__ __forceinline__ float2v swap32(float v) {
-    const uint32_t a = __builtin_bit_cast(uint32_t, v);
-    return __builtin_bit_cast(float2v, __builtin_amdgcn_permlane32_swap(a, a, false, false));
-}
-__device__ __forceinline__ float quarters_max(float v) {
-    const float2v r = swap16(v);
-    const float2v s = swap32(fmaxf(r[0], r[1]));
-    return fmaxf(s[0], s[1]);
-}
-__device__ __forceinline__ float quarters_sum(float v) {
-    const float2v r = swap16(v);
-    const float2v s = swap32(r[0] + r[1]);
-    return s[0] + s[1];
-}
 
 __global__ __launch_bounds__(kSplitThreads, 2) void decode_split_kernel(DecodeSplitArgs a) {
     __shared__ __attribute__((aligned(16))) float so[kSplitWaves][kAttnMaxGroup][kOutStride];
@@ -141,31 +118,8 @@ __global__ __launch_bounds__(kSplitThreads, 2) void decode_split_kernel(DecodeSp
     Kv buf[2];
     if (blk < blocks) load(buf[0], blk);
 
-    // A rotated head vector as operand pieces: dimensions 32 s + 8 q .. + 7,
-    // whose rotate_half partners are piece s ^ 2 of the same lane.  Each
-    // product and the sum is rounded to bf16 (model.py:17-19, :76-77).
-    auto rope = [&](const uint16_t* vec, u32x4 (&r)[4]) {
-        u32x4 x[4], c[4], n[4];
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            x[s] = *(const u32x4*)(vec + 32 * s + 8 * q);
-            c[s] = *(const u32x4*)(cs + 32 * s + 8 * q);
-            n[s] = *(const u32x4*)(sn + 32 * s + 8 * q);
-        }
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const float sign = s < 2 ? -1.0f : 1.0f;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t pa = pack_bf16x2(bf16_lo(x[s][e]) * bf16_lo(c[s][e]), bf16_hi(x[s][e]) * bf16_hi(c[s][e]));
-                const uint32_t pb = pack_bf16x2((sign * bf16_lo(x[s ^ 2][e])) * bf16_lo(n[s][e]),
-                                                (sign * bf16_hi(x[s ^ 2][e])) * bf16_hi(n[s][e]));
-                r[s][e] = pack_bf16x2(bf16_lo(pa) + bf16_lo(pb), bf16_hi(pa) + bf16_hi(pb));
-            }
-        }
-    };
     u32x4 qf[4];  // columns past the group repeat its last head and are not stored
-    rope(qkv + (kvh * group + min(j, group - 1)) * kAttnHeadDim, qf);
+    rope_pieces(qkv + (kvh * group + min(j, group - 1)) * kAttnHeadDim, cs, sn, q, qf);
 
     float m_run = -INFINITY, l_run = 0.0f;
     float4v o[8];
@@ -180,7 +134,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void decode_split_kernel(DecodeSp
             const u32x4 vnew = *(const u32x4*)(qkv + (a.heads + a.kv_heads + kvh) * kAttnHeadDim + 8 * j);
             const u32x4 zero = {0u, 0u, 0u, 0u};
             u32x4 kf[4];
-            rope(qkv + (a.heads + kvh) * kAttnHeadDim, kf);
+            rope_pieces(qkv + (a.heads + kvh) * kAttnHeadDim, cs, sn, q, kf);
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
                 const bool here = t0 + 16 * m + j == pos;

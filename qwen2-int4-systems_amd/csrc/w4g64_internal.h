@@ -159,6 +159,24 @@ constexpr int kDecodeMaxSplits = 64;
 int decode_splits(int64_t batch, int64_t kv_heads, int64_t max_length);
 hipError_t launch_decode_split(const DecodeSplitArgs& args, int64_t batch, hipStream_t stream);
 
+// Prompt attention (qwen2_prefill.hip).
+struct PrefillArgs {
+    const uint16_t* qkv;  // [batch * length][(heads + 2 kv_heads) * 128]
+    const uint16_t* cos;  // [batch * length][128]
+    const uint16_t* sin;
+    uint16_t* k_cache;    // [batch][kv_heads][max_len][128]
+    uint16_t* v_cache;
+    uint16_t* out;        // [batch * length][heads * 128]
+    int batch;
+    int length;
+    int heads;
+    int kv_heads;
+    int max_len;
+    float scale2;         // |scale| * log2(e): the softmax runs in base 2
+    uint32_t query_sign;  // sign bits of two bf16 queries, set for a negative scale
+};
+hipError_t launch_prefill_attention(const PrefillArgs& args, hipStream_t stream);
+
 // Chunks the attention-merge form of the pipelined GEMV takes (the cache's
 // max_length up to 1024 positions): it loads every chunk's partial result.
 constexpr int kAttnMergeMaxChunks = 16;

@@ -398,6 +398,57 @@ def test_prefill_attention_matches_torch(batch, heads, kv_heads, length, max_len
     assert cos_sim.item() >= 0.99999, cos_sim.item()
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,length,max_length,scale,shift", [
+    (1, 12, 2, 31, 31, 128 ** -0.5, 0),    # the cache ends with the prompt, a partial block
+    (2, 3, 3, 32, 40, 128 ** -0.5, 1),     # exactly one block; factors and output only 2-byte aligned
+    (1, 8, 1, 33, 64, -0.05, 0),           # one row past a block; a negative scale
+    (1, 2, 2, 160, 161, 128 ** -0.5, 0),   # five blocks: one wave takes two
+    (1, 14, 2, 1021, 1024, 1.0, 3),        # sharp softmax: rows rescaled late, many blocks per wave
+])
+def test_prefill_attention_block_edges(batch, heads, kv_heads, length, max_length, scale, shift):
+    """qwen2_prefill_attention at the edges of its 32-row tiles and 32-key
+    blocks against the same in fp64 from the rounded rotary step: fp32 scores
+    of magnitude up to s carry an error of about 128 2^-24 s into the
+    exponent, so an output differs by at most its bf16 rounding (2^-8 of the
+    value) plus (2^-16 + 2^-16 s) of the largest one."""
+    lib = _lib.load()
+    g = _gen(batch * 100 + length)
+    d, rows = 128, batch * length
+    qkv = torch.randn((rows, (heads + 2 * kv_heads) * d), generator=g, device="cuda").to(torch.bfloat16)
+    caches = torch.randn((2, batch, kv_heads, max_length, d), generator=g, device="cuda").to(torch.bfloat16)
+    k_cache, v_cache = caches.clone().unbind(0)
+    positions = torch.arange(length, device="cuda").repeat(batch)
+
+    def shifted(cols):  # a tensor that starts `shift` elements into its storage
+        return torch.empty(rows * cols + shift, dtype=torch.bfloat16, device="cuda")[shift:].view(rows, cols)
+
+    cos, sin, out = shifted(d), shifted(d), shifted(heads * d)
+    for to, value in zip((cos, sin), RotaryEmbedding(d, 1_000_000.0).cuda()(positions, torch.bfloat16)):
+        to.copy_(value)
+    ws = torch.empty(lib.qwen2_prefill_attention_workspace_bytes(batch, heads, length), dtype=torch.uint8,
+                     device="cuda")
+    _lib.check(lib.qwen2_prefill_attention(
+        _p(qkv), _p(cos), _p(sin), _p(k_cache), _p(v_cache), _p(out), batch, length, heads, kv_heads, d, max_length,
+        ctypes.c_float(scale), _p(ws), ws.numel(), _stream()))
+    torch.cuda.synchronize()
+    q, k, v = (t.view(batch, length, -1, d).transpose(1, 2)
+               for t in qkv.split([heads * d, kv_heads * d, kv_heads * d], dim=1))
+    c, s = cos.view(batch, 1, length, d), sin.view(batch, 1, length, d)
+    q, k = q * c + rotate_half(q) * s, k * c + rotate_half(k) * s
+    want_k, want_v = caches.clone().unbind(0)
+    want_k[:, :, :length], want_v[:, :, :length] = k, v
+    assert torch.equal(k_cache, want_k) and torch.equal(v_cache, want_v)
+    group = heads // kv_heads
+    k, v = (t.double().repeat_interleave(group, dim=1) for t in (k, v))
+    scores = torch.matmul(q.double(), k.transpose(-1, -2).contiguous()) * scale
+    causal = torch.ones((length, length), dtype=torch.bool, device="cuda").tril()
+    probs = torch.softmax(scores.masked_fill(~causal, float("-inf")), dim=-1)
+    want = torch.matmul(probs, v).transpose(1, 2).reshape(rows, heads * d)
+    err = (out.double() - want).abs()
+    bound = want.abs() * 2.0 ** -8 + want.abs().max() * 2.0 ** -16 * (1 + scores.abs().max())
+    assert bool((err <= bound).all()), (err - bound).max().item()
+
+
 @pytest.mark.parametrize("rows,inter", [(1, 8960), (4, 8960), (16, 100)])
 def test_silu_mul_matches_torch(rows, inter):
     lib = _lib.load()
