@@ -270,9 +270,11 @@ static int linear_impl(const void* x, int x_dtype, const uint8_t* qweight, const
     if (!w4g64::gemm_supported(p))
         return fail(W4G64_STATUS_UNSUPPORTED, "GEMM path supports rows * in_features below 2^31 (2^30 for float32) "
                     "and out_features * in_features below 2^32");
-    const int64_t need = w4g64::gemm_workspace_bytes(rows, out_features, in_features, x_dtype);
+    const int64_t need = w4g64::gemm_least_workspace_bytes(rows, out_features, in_features, x_dtype);
     if (int st = check_workspace(workspace, workspace_bytes, need)) return st;
-    return hip_status(w4g64::launch_gemm(p, workspace, s, (hipEvent_t)start_event, (hipEvent_t)stop_event), "gemm");
+    return hip_status(w4g64::launch_gemm(p, workspace, workspace_bytes, s, (hipEvent_t)start_event,
+                                         (hipEvent_t)stop_event),
+                      "gemm");
 }
 
 int w4g64_linear(const void* x, int x_dtype, const uint8_t* qweight, const uint16_t* scales, const uint8_t* zeros,
@@ -353,9 +355,9 @@ int w4g64_linear_swiglu(const void* gate_up, const uint8_t* qweight, const uint1
         if (!w4g64::gemm_supported(p))
             return fail(W4G64_STATUS_UNSUPPORTED, "GEMM path supports rows * in_features below 2^30 and "
                         "out_features * in_features below 2^32");
-        const int64_t need = w4g64::gemm_workspace_bytes(rows, out_features, in_features, w4g64::kSwiGLU);
+        const int64_t need = w4g64::gemm_least_workspace_bytes(rows, out_features, in_features, w4g64::kSwiGLU);
         if (int st = check_workspace(workspace, workspace_bytes, need)) return st;
-        return hip_status(w4g64::launch_gemm(p, workspace, (hipStream_t)stream), "gemm");
+        return hip_status(w4g64::launch_gemm(p, workspace, workspace_bytes, (hipStream_t)stream), "gemm");
     }
     const w4g64::GemvPlan plan = w4g64::plan_gemv(rows, out_features, in_features, w4g64::kSwiGLU);
     if (int st = check_workspace(workspace, workspace_bytes, plan.workspace_bytes)) return st;

@@ -53,8 +53,8 @@
 //   * Tiles are assigned so that the workgroups of one XCD (ids congruent
 //     mod 8) cover consecutive tiles of one row band: they share the
 //     activation band in their L2.
-#include "w4g64_device.h"
 #include "w4g64_internal.h"
+#include "w4g64_gemm.h"
 
 namespace w4g64 {
 namespace {
@@ -89,8 +89,6 @@ struct GemmArgs {
 };
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
-// Word 3 of a raw gfx9 buffer resource (32-bit data format; no swizzle, no stride).
-constexpr int kRsrcWord3 = 0x00020000;
 
 // s_waitcnt with only the vector memory counter constrained (gfx9 encoding:
 // vmcnt bits [3:0] and [15:14], expcnt [6:4] and lgkmcnt [11:8] left at max).
@@ -112,31 +110,6 @@ __device__ __forceinline__ void block_barrier() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-}
-
-// Bitwise select (x ^ C) & M | (C & ~M), one v_bitop3: inside the mask the
-// nibble n XOR 8 = n' = code + 8, outside it the magic exponent bits of C.
-template <uint32_t C, uint32_t M>
-__device__ __forceinline__ uint32_t nib_select(uint32_t x) {
-    return ((x ^ C) & M) | (C & ~M);
-}
-// fp16 pairs (1024 + n', 1024 + n'') from bits 0-3 / 16-19 and (64 + n', 64 +
-// n'') from bits 4-7 / 20-23 (n' XOR-ed in by the 8s of C).
-constexpr uint32_t kMaskLo = 0x000F000Fu, kSelLo = 0x64086408u;
-constexpr uint32_t kMaskHi = 0x00F000F0u, kSelHi = 0x54805480u;
-
-// (code - zero) of one packed dword (8 consecutive K values of a column), as
-// 4 fp16 pairs in slot order [k0 k4 | k1 k5 | k2 k6 | k3 k7].  zlo = fp16
-// pair (1032 + z, 1032 + z), zhi = (72 + z, 72 + z): (1024 + n') - (1032 + z)
-// = (64 + n') - (72 + z) = code - z, exact.
-__device__ __forceinline__ u32x4 decode_codes(uint32_t w, half2v zlo, half2v zhi) {
-    const uint32_t w8 = w >> 8;
-    u32x4 r;
-    r[0] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, nib_select<kSelLo, kMaskLo>(w)) - zlo);
-    r[1] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, nib_select<kSelHi, kMaskHi>(w)) - zhi);
-    r[2] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, nib_select<kSelLo, kMaskLo>(w8)) - zlo);
-    r[3] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, nib_select<kSelHi, kMaskHi>(w8)) - zhi);
-    return r;
 }
 
 // Tile t -> (row band, column tile): bands in groups of bg, each group's
@@ -668,69 +641,11 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmArgs a) {
 // [2^14, 2^15); fp16 input keeps e = 0 -- and stored as fp16 (two planes for
 // the fp32-class kinds: hi = RNE(t) and lo = RNE(t - hi)), each 8-value chunk
 // in slot order [k0 k4 k1 k5 k2 k6 k3 k7]; rowscale[m] = 2^e.
-template <int XK>
-__device__ __forceinline__ void stage_load8(const void* x, int64_t m, int K, int c, float (&v)[8]) {
-    if constexpr (XK == kF16 || XK == kBF16) {
-        const u32x4 d = *(const u32x4*)((const uint16_t*)x + m * K + 8 * c);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t bits = (d[i / 2] >> (16 * (i & 1))) & 0xFFFFu;
-            v[i] = XK == kF16 ? half_bits_to_float((uint16_t)bits) : bf16_bits_to_float(bits);
-        }
-    } else if constexpr (XK == kF32) {
-        const float4v f0 = *(const float4v*)((const float*)x + m * K + 8 * c);
-        const float4v f1 = *(const float4v*)((const float*)x + m * K + 8 * c + 4);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[i] = f0[i];
-            v[4 + i] = f1[i];
-        }
-    } else {
-        const uint16_t* gu = (const uint16_t*)x + m * 2 * K + 8 * c;
-        const u32x4 gv = *(const u32x4*)gu;
-        const u32x4 uv = *(const u32x4*)(gu + K);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float gf = bf16_bits_to_float((gv[i / 2] >> (16 * (i & 1))) & 0xFFFFu);
-            const float uf = bf16_bits_to_float((uv[i / 2] >> (16 * (i & 1))) & 0xFFFFu);
-            v[i] = (gf / (1.0f + expf(-gf))) * uf;
-        }
-    }
-}
-
-// Scale 2^-e for a row whose largest finite magnitude is mx (e = 0 for 0).
-__device__ __forceinline__ void row_factors(float mx, float& inv, float& rs) {
-    inv = 1.0f;
-    rs = 1.0f;
-    if (mx > 0.0f) {
-        int ex;
-        (void)frexpf(mx, &ex);  // mx = f 2^ex, f in [0.5, 1)
-        int sh = 15 - ex;       // mx 2^sh in [2^14, 2^15)
-        sh = sh > 126 ? 126 : sh;
-        inv = ldexpf(1.0f, sh);
-        rs = ldexpf(1.0f, -sh);
-    }
-}
-
 // Chunk c of the staged row: the 8 values times inv, as fp16 hi (and lo) in slot order.
 template <bool kTwo>
 __device__ __forceinline__ void stage_store8(uint16_t* row_out, int K, int c, const float (&v)[8], float inv) {
-    constexpr int kSlot[8] = {0, 4, 1, 5, 2, 6, 3, 7};
     u32x4 hi, lo;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        uint32_t hb[2], lb[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const float t = v[kSlot[2 * p + h]] * inv;
-            const _Float16 th = (_Float16)t;
-            hb[h] = __builtin_bit_cast(uint16_t, th);
-            // (an infinite hi keeps a zero lo: inf - inf would turn the row's results into NaN)
-            lb[h] = __builtin_isfinite((float)th) ? __builtin_bit_cast(uint16_t, (_Float16)(t - (float)th)) : 0;
-        }
-        hi[p] = hb[0] | (hb[1] << 16);
-        lo[p] = lb[0] | (lb[1] << 16);
-    }
+    stage_split8(v, inv, hi, lo);
     *(u32x4*)(row_out + 8 * c) = hi;
     if constexpr (kTwo) *(u32x4*)(row_out + K + 8 * c) = lo;
 }
@@ -886,10 +801,24 @@ GemmLayout gemm_layout(int64_t rows, int64_t out_features, int64_t in_features, 
     return l;
 }
 
+// Few row tiles have a kernel of their own, faster at every size measured up to
+// its limits (w4g64_gemm_rows.hip), where the workspace holds its plan.  The
+// tiled plan's bytes stay what a call must bring, and what the workspace query
+// answers unless the other plan needs a little more (rows padded to 32, short
+// K), so that no caller's scratch (w4g64_linear_static_scratch among them)
+// becomes too small or is suddenly large enough.
+constexpr int64_t kFewRowsExtra = 1 << 20;
+
 }  // namespace
 
-int64_t gemm_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
+int64_t gemm_least_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
     return gemm_layout(rows, out_features, in_features, x_kind).bytes;
+}
+
+int64_t gemm_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
+    const int64_t tiled = gemm_least_workspace_bytes(rows, out_features, in_features, x_kind);
+    const RowsPlan few = plan_rows(rows, out_features, in_features, x_kind);
+    return few.taken && few.workspace_bytes > tiled && few.workspace_bytes <= kFewRowsExtra ? few.workspace_bytes : tiled;
 }
 
 bool gemm_supported(const LinearProblem& p) {
@@ -900,7 +829,15 @@ bool gemm_supported(const LinearProblem& p) {
 }
 
 const char* gemm_kernel_name(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
-    const bool eight = gemm_eight_waves(gemm_layout(rows, out_features, in_features, x_kind).plan);
+    const GemmLayout l = gemm_layout(rows, out_features, in_features, x_kind);
+    const RowsPlan few = plan_rows(rows, out_features, in_features, x_kind);
+    if (few.taken && few.workspace_bytes <= (l.bytes > kFewRowsExtra ? l.bytes : kFewRowsExtra)) {
+        if (x_kind == kF16) return "gemm_kernel<f16 a x int b,few rows> (fp16 rows staged)";
+        if (x_kind == kBF16) return "gemm_kernel<f16 a x int b,few rows> (bf16 rows staged as scaled fp16)";
+        if (x_kind == kSwiGLU) return "gemm_kernel<f16 a x int b,few rows> (silu(gate)*up staged as scaled fp16 hi|lo)";
+        return "gemm_kernel<f16 a x int b,few rows> (f32 rows staged as scaled fp16 hi|lo)";
+    }
+    const bool eight = gemm_eight_waves(l.plan);
     if (x_kind == kF16)
         return eight ? "gemm_kernel<f16 a x int b,128x256,8 waves> (fp16 rows staged)"
                      : "gemm_kernel<f16 a x int b,128x256> (fp16 rows staged)";
@@ -914,8 +851,10 @@ const char* gemm_kernel_name(int64_t rows, int64_t out_features, int64_t in_feat
                  : "gemm_kernel<f16 a x int b,128x256> (f32 rows staged as scaled fp16 hi|lo)";
 }
 
-hipError_t launch_gemm(const LinearProblem& p, void* workspace, hipStream_t stream, hipEvent_t start,
-                       hipEvent_t stop) {
+hipError_t launch_gemm(const LinearProblem& p, void* workspace, int64_t workspace_bytes, hipStream_t stream,
+                       hipEvent_t start, hipEvent_t stop) {
+    const RowsPlan few = plan_rows(p.rows, p.out_features, p.in_features, p.x_kind);
+    if (few.taken && few.workspace_bytes <= workspace_bytes) return launch_rows(p, few, workspace, stream, start, stop);
     const GemmLayout l = gemm_layout(p.rows, p.out_features, p.in_features, p.x_kind);
     const GemmPlan& pl = l.plan;
     const bool two = two_planes(p.x_kind);

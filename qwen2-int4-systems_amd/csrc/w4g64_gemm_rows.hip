@@ -1,0 +1,491 @@
+// W4G64 GEMM for a few row tiles (17 to 128 rows; fp32-class activations to
+// 64): batched decode, draft verification, short prompts.  The arithmetic is
+// the prefill GEMM's (w4g64_gemm.hip): staged fp16 rows times a power of two,
+// exact integer (code - zero) on the matrix cores, the group scale in fp32,
+// the row factor last.  What differs is the shape: a 128 x 256 tile is mostly
+// padding there, and its few tiles need a K split and a reduction launch to
+// fill the chip.
+//
+//   rows_stage_kernel, rows_stage_swiglu_kernel
+//       fp16 values (hi and lo planes for the fp32-class kinds) in MFMA
+//       operand order [row tile][group][plane][half][lane][8], so that an
+//       operand load is a contiguous kilobyte.
+//   rows_gemm_kernel
+//       one workgroup of W waves per 16 CT output features and K range.  Each
+//       wave takes a contiguous part of the range's groups over all rows;
+//       the waves' sums meet in LDS at the end.  Two planes meet the same
+//       decoded weights, in one sum per group.
+//
+// Bound by vector memory instructions: one that reads a few bytes of 16 rows
+// costs a cache line per lane where one over contiguous lanes costs four.
+// With weights, scales and zero points loaded straight into operands gate|up
+// 17920x1536 at 24 rows spent 15 us here, 63 cycles per load; with the weights
+// by 64-byte runs through the wave's own LDS and the scales staged once per
+// workgroup, 8.  Per call with the staging and any reduction, bf16,
+// graph-replayed over rotated weights, against the 128 x 256 tiles: 24 x
+// 17920x1536 29.0 -> 11.6 us, 24 x 1536x1536 16.0 -> 6.8, 40 x 8960x1536 23.1
+// -> 11.1, 128 x 8960x1536 27.9 -> 19.2, 24 x 1536x8960 of the SwiGLU
+// product (fp32) 33.2 -> 16.1, 64 x 1536x8960 fp32 32.7 -> 22.4.
+#include "w4g64_gemm.h"
+#include "w4g64_internal.h"
+
+namespace w4g64 {
+namespace {
+
+struct RowsArgs {
+    const uint16_t* x;      // staged rows, operand order
+    const float* rowscale;  // power-of-two row factors
+    const uint8_t* qweight;
+    const uint16_t* scales;
+    const uint8_t* zeros;
+    const void* bias;
+    int bias_kind;
+    void* y;
+    int out_kind;
+    float* partials;  // [splits][M][N], or null
+    int M;
+    int N;
+    int G;    // groups
+    int gps;  // groups per K range, even
+    int const_bytes;
+    int vec_out;  // y is 16-byte aligned and N % 4 == 0
+};
+
+// Operand slot (16-byte unit) of row m, chunk c (8 values, K = 8 c .. 8 c + 7)
+// of a plane: [row tile][group][plane][half][lane].
+template <int PL>
+__device__ __forceinline__ int64_t operand_slot(int m, int c, int plane, int G) {
+    return (((((int64_t)(m >> 4) * G + (c >> 3)) * PL + plane) * 2 + (c & 1)) * 64) + ((c >> 1) & 3) * 16 + (m & 15);
+}
+
+// Workgroup barrier that covers LDS alone: global loads stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int XK, int THREADS>
+__global__ __launch_bounds__(THREADS) void rows_stage_kernel(const void* x, u32x4* out, float* rowscale, int K) {
+    constexpr int kPlanes = XK == kF32 ? 2 : 1;
+    constexpr int kHeld = 2;
+    __shared__ float wmax[THREADS / 64];
+    const int m = blockIdx.x;
+    const int chunks = K / 8;
+    const int G = K / 64;
+    float v[kHeld][8];
+    float mx = 0.0f;
+    auto largest = [&](const float (&t)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (__builtin_isfinite(t[i])) mx = fmaxf(mx, fabsf(t[i]));
+    };
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        const int c = threadIdx.x + THREADS * u;
+        if (c < chunks) {
+            stage_load8<XK>(x, m, K, c, v[u]);
+            largest(v[u]);
+        }
+    }
+    for (int c = threadIdx.x + THREADS * kHeld; c < chunks; c += THREADS) {  // (read again below)
+        float t[8];
+        stage_load8<XK>(x, m, K, c, t);
+        largest(t);
+    }
+    float inv = 1.0f, rs = 1.0f;
+    if constexpr (XK != kF16) {
+        mx = wave_max64(mx);
+        if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < THREADS / 64; ++w) mx = fmaxf(mx, wmax[w]);
+        row_factors(mx, inv, rs);
+    }
+    if (threadIdx.x == 0) rowscale[m] = rs;
+    auto store = [&](int c, const float (&t)[8]) {
+        u32x4 hi, lo;
+        stage_split8(t, inv, hi, lo);
+        out[operand_slot<kPlanes>(m, c, 0, G)] = hi;
+        if constexpr (kPlanes == 2) out[operand_slot<kPlanes>(m, c, 1, G)] = lo;
+    };
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+        const int c = threadIdx.x + THREADS * u;
+        if (c < chunks) store(c, v[u]);
+    }
+    for (int c = threadIdx.x + THREADS * kHeld; c < chunks; c += THREADS) {
+        float t[8];
+        stage_load8<XK>(x, m, K, c, t);
+        store(c, t);
+    }
+}
+
+// The SwiGLU product, one workgroup per row and 2048 values: its exponentials
+// and divisions, on one CU per row, took 7.0 us at 24 x 8960.  Every
+// workgroup of a row scans all of it for the largest finite |gate| and |up|,
+// whose exponents bound the product's (|silu(g)| <= |g|), so they agree on the
+// row's factor; the few bits by which the bound is too large come off a range
+// of 2^-24 below 2^15.
+__global__ __launch_bounds__(256) void rows_stage_swiglu_kernel(const void* x, u32x4* out, float* rowscale, int K) {
+    __shared__ uint32_t wmax[2][4];
+    const int m = blockIdx.x;
+    const int chunks = K / 8;
+    const uint16_t* gu = (const uint16_t*)x + (int64_t)m * 2 * K;
+    const int own = blockIdx.y * 256 + threadIdx.x;
+    float v[8];
+    if (own < chunks) stage_load8<kSwiGLU>(x, m, K, own, v);
+    uint32_t mx[2] = {0, 0};  // bf16 magnitude bits
+    for (int c = threadIdx.x; c < chunks; c += 256) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const u32x4 d = *(const u32x4*)(gu + (int64_t)p * K + 8 * c);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t lo = d[i] & 0x7FFFu, hi = (d[i] >> 16) & 0x7FFFu;
+                mx[p] = max(mx[p], max(lo < 0x7F80u ? lo : 0u, hi < 0x7F80u ? hi : 0u));
+            }
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        // (magnitude bits of non-negative bf16 values order as the values do)
+        const float w = wave_max64(bf16_bits_to_float(mx[p]));
+        if ((threadIdx.x & 63) == 0) wmax[p][threadIdx.x >> 6] = __builtin_bit_cast(uint32_t, w);
+    }
+    __syncthreads();
+    int e = 0;
+    bool zero = false;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const float w = __builtin_bit_cast(float, max(max(wmax[p][0], wmax[p][1]), max(wmax[p][2], wmax[p][3])));
+        int ex;
+        (void)frexpf(w, &ex);  // w = f 2^ex, f in [0.5, 1)
+        e += ex;
+        zero = zero || w == 0.0f;
+    }
+    // products lie below 2^e; a finite one below 2^128
+    float inv, rs;
+    row_factors(zero ? 0.0f : ldexpf(0.5f, max(min(e, 128), -125)), inv, rs);
+    if (threadIdx.x == 0 && blockIdx.y == 0) rowscale[m] = rs;
+    if (own < chunks) {
+        u32x4 hi, lo;
+        stage_split8(v, inv, hi, lo);
+        out[operand_slot<2>(m, own, 0, K / 64)] = hi;
+        out[operand_slot<2>(m, own, 1, K / 64)] = lo;
+    }
+}
+
+template <int PL, int MT, int CT, int W>
+__global__ __launch_bounds__(64 * W) void rows_gemm_kernel(RowsArgs a) {
+    constexpr int kRows = 16 * MT, kCols = 16 * CT;
+    constexpr int kStride = kCols + 4;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15;
+    const int q = lane >> 4;
+    const int n0 = blockIdx.x * kCols;
+    const int first = blockIdx.y * a.gps;  // (gps is even)
+    const int count = min(a.gps, a.G - first);
+    const int pairs = (count + 1) / 2;
+    const int beg = first + 2 * (pairs * wave / W);  // this wave's groups: whole pairs
+    const int end = min(first + 2 * (pairs * (wave + 1) / W), first + count);
+    // LDS: per group of the range and column the scale and the zero point's
+    // constants; per wave CT kilobytes of packed weights
+    u32x2* consts = (u32x2*)smem;
+    unsigned char* mine = smem + a.const_bytes + 1024 * CT * wave;
+
+    const __amdgpu_buffer_rsrc_t x_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)((uint32_t)(MT * a.G) * (2048u * PL)), kRsrcWord3);
+    const __amdgpu_buffer_rsrc_t w_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a.qweight, 0, (int)((uint32_t)a.N * (uint32_t)a.G * 32u), kRsrcWord3);
+
+    // ---- scales and zero points: a column's groups by consecutive lanes ----
+    constexpr int kOwn = (kCols + W - 1) / W;
+    for (int g0 = 0; g0 < count; g0 += 64) {
+        const int g = min(g0 + lane, count - 1);
+        uint32_t sv[kOwn], zv[kOwn];
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) {
+            const uint32_t e = (uint32_t)min(n0 + wave + W * i, a.N - 1) * (uint32_t)a.G + (uint32_t)(first + g);
+            sv[i] = a.scales[e];
+            zv[i] = (uint32_t)a.zeros[e >> 1] >> (4 * (e & 1));
+        }
+#pragma unroll
+        for (int i = 0; i < kOwn; ++i) {
+            const int zn = __builtin_amdgcn_sbfe((int)zv[i], 0, 4);
+            // fp16 bits of 1032 + z (mantissa unit 1) and of 72 + z (mantissa unit 1/16)
+            if (g0 + lane < count && wave + W * i < kCols)
+                consts[(g0 + lane) * kCols + wave + W * i] =
+                    u32x2{__builtin_bit_cast(uint32_t, half_bits_to_float((uint16_t)sv[i])),
+                          (uint32_t)(0x6408 + zn) | ((uint32_t)(0x5480 + 16 * zn) << 16)};
+        }
+    }
+
+    // Packed weights of a pair of groups, 64 bytes of a column: four
+    // consecutive lanes load it (operand form straight from memory would be 8
+    // bytes of 16 rows per 16 lanes, a cache line each), and it goes through
+    // the wave's own LDS.  Piece c of column r in slot c ^ (r / 4 % 4): the
+    // 8-byte operand reads of 16 columns meet different banks.
+    uint32_t w_at[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+        w_at[c] = (uint32_t)min(n0 + 16 * c + (lane >> 2), a.N - 1) * (uint32_t)a.G * 32u + 16u * (lane & 3);
+    unsigned char* w_put = mine + 64 * (lane >> 2) + 16 * ((lane & 3) ^ ((lane >> 4) & 3));
+    const unsigned char* w_get[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) w_get[u] = mine + 64 * j + 16 * ((2 * u + (q >> 1)) ^ (j >> 2)) + 8 * (q & 1);
+
+    struct Rows {
+        u32x4 x[MT][PL][2];
+    };
+    auto load_w = [&](u32x4 (&w)[CT], int g) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+            w[c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_at[c], 32 * g, 0));
+    };
+    auto load_x = [&](Rows& t, int g) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int p = 0; p < PL; ++p)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    t.x[m][p][h] = __builtin_bit_cast(
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, 16 * lane + 1024 * (2 * p + h),
+                                                                     2048 * PL * (m * a.G + g), 0));
+    };
+    float4v acc[MT][CT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[m][c] = float4v{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const Rows& t, int g, int u) {  // u: the group's half of its pair
+        u32x4 f[CT][2];
+        float sc[CT];
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            const u32x2 w = *(const u32x2*)(w_get[u] + 1024 * c);
+            const u32x2 k = consts[(g - first) * kCols + 16 * c + j];
+            const uint32_t scale = k[0], zero = k[1];  // (a bit cast of a vector's element reads element 0)
+            sc[c] = __builtin_bit_cast(float, scale);
+            const half2v z = __builtin_bit_cast(half2v, zero);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) f[c][h] = decode_codes(w[h], half2v{z[0], z[0]}, half2v{z[1], z[1]});
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                float4v d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int p = 0; p < PL; ++p)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, t.x[m][p][h]),
+                                                                   __builtin_bit_cast(half8, f[c][h]), d, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[m][c][r] = __builtin_fmaf(sc[c], d[r], acc[m][c][r]);
+            }
+    };
+    auto put_w = [&](const u32x4 (&w)[CT]) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c) *(u32x4*)(w_put + 1024 * c) = w[c];
+    };
+    Rows x0, x1;
+    u32x4 w[CT];
+    if (beg < end) {
+        load_w(w, beg);
+        load_x(x0, beg);
+        load_x(x1, min(beg + 1, end - 1));
+    }
+    lds_barrier();  // the constants are in place (loads stay in flight)
+    if (beg < end) {
+        int g = beg;
+        for (; g + 2 < end; g += 2) {
+            put_w(w);
+            load_w(w, g + 2);
+            compute(x0, g, 0);
+            load_x(x0, g + 2);
+            compute(x1, g + 1, 1);
+            load_x(x1, min(g + 3, end - 1));
+        }
+        put_w(w);
+        compute(x0, g, 0);
+        if (g + 1 < end) compute(x1, g + 1, 1);
+    }
+
+    // ---- the waves' sums meet in LDS, added in wave order ----
+    lds_barrier();
+    float(*so)[kRows][kStride] = (float(*)[kRows][kStride])smem;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) so[wave][16 * m + 4 * q + r][16 * c + j] = acc[m][c][r];
+    __syncthreads();
+    for (int e = tid; e < kRows * kCols / 4; e += 64 * W) {
+        const int row = e / (kCols / 4);
+        const int col = 4 * (e % (kCols / 4));
+        const int n = n0 + col;
+        if (row >= a.M || n >= a.N) continue;
+        float4v sum = *(const float4v*)&so[0][row][col];
+#pragma unroll
+        for (int w = 1; w < W; ++w) sum += *(const float4v*)&so[w][row][col];
+        sum *= a.rowscale[row];
+        const int64_t at = (int64_t)row * a.N + n;
+        if (a.partials) {
+            float* to = a.partials + (int64_t)blockIdx.y * a.M * a.N + at;
+            for (int i = 0; i < 4 && n + i < a.N; ++i) to[i] = sum[i];
+            continue;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum[i] += load_bias(a.bias, a.bias_kind, n + i < a.N ? n + i : a.N - 1);
+        if (PL == 2 || a.out_kind == kF32) {
+            float* to = (float*)a.y + at;
+            if (a.vec_out) *(float4v*)to = sum;
+            else
+                for (int i = 0; i < 4 && n + i < a.N; ++i) to[i] = sum[i];
+            continue;
+        }
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = a.out_kind == kF16 ? float_to_half_bits(sum[i]) : float_to_bf16_bits(sum[i]);
+        uint16_t* to = (uint16_t*)a.y + at;
+        if (a.vec_out) *(u32x2*)to = u32x2{v[0] | (v[1] << 16), v[2] | (v[3] << 16)};
+        else
+            for (int i = 0; i < 4 && n + i < a.N; ++i) to[i] = (uint16_t)v[i];
+    }
+}
+
+bool two_planes(int x_kind) { return x_kind == kF32 || x_kind == kSwiGLU; }
+
+}  // namespace
+
+// Waves and columns per workgroup, K ranges.  Measured per call (24, 40, 64
+// and 96 rows; CT x W with one range, or with the ranges given):
+//   up to 256 column tiles, K up to 4096: 1 x 8 (2048x1536 at 24 rows 7.0 us
+//     against 7.2 for 1 x 4 and 7.6 for 2 x 8; 4096x4096 at 40 11.0, 11.7, 12.3);
+//   more column tiles: 1 x 4 while they are few enough to be one round of
+//     workgroups (8960x1536 at 40 rows 11.1, 2 x 4 11.6; 17920x1536 at 24 12.0,
+//     2 x 4 11.6) and the rows' loads do not dominate (96 rows 16.8, 2 x 4 15.9);
+//   longer K: 2 x 8 and as many ranges as keep one workgroup per CU
+//     (1536x8960 at 40 rows: one range 17.0, two of 1 x 8 15.0, four of 2 x 8
+//     14.7).
+// A range holds at most 160 groups (40 KB of scales and zero points in LDS).
+RowsPlan plan_rows(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
+    RowsPlan pl{};
+    const bool two = two_planes(x_kind);
+    const int64_t tiles = (rows + 15) / 16;
+    if (tiles < 2 || tiles > (two ? 4 : 8)) return pl;
+    pl.tiles = (int)(tiles == 5 ? 6 : (tiles == 7 ? 8 : tiles));
+    const int64_t staged = (int64_t)pl.tiles * 16 * in_features * (two ? 4 : 2);
+    if (staged >= (int64_t(1) << 31)) return pl;  // 32-bit operand offsets
+    const int G = (int)(in_features / 64);
+    const int64_t columns = (out_features + 15) / 16;
+    pl.cols = 1;
+    pl.waves = 8;
+    int64_t splits = 1;
+    if (G > 64) {
+        pl.cols = 2;
+        splits = 224 / ((columns + 1) / 2);
+        splits = splits < G / 16 ? splits : G / 16;
+    } else if (columns > 256) {
+        pl.cols = columns <= 640 && tiles <= 4 ? 1 : 2;
+        pl.waves = 4;
+    }
+    const int64_t least = (G + 159) / 160;
+    splits = splits < least ? least : splits;
+    pl.gps = (int)((G + splits - 1) / splits + 1) / 2 * 2;
+    pl.splits = (G + pl.gps - 1) / pl.gps;
+    auto up256 = [](int64_t v) { return (v + 255) / 256 * 256; };
+    pl.staged_offset = up256(pl.splits > 1 ? (int64_t)pl.splits * rows * out_features * 4 : 0);
+    pl.rowscale_offset = pl.staged_offset + up256(staged);
+    pl.workspace_bytes = pl.rowscale_offset + rows * 4;
+    pl.taken = true;
+    return pl;
+}
+
+namespace {
+template <int PL, int MT, int CT, int W>
+hipError_t launch_shape(RowsArgs args, const RowsPlan& pl, hipStream_t stream, hipEvent_t stop) {
+    args.const_bytes = args.gps * 16 * CT * 8;
+    const dim3 grid((unsigned)((args.N + 16 * CT - 1) / (16 * CT)), (unsigned)pl.splits);
+    const size_t sums = (size_t)W * (16 * MT) * (16 * CT + 4) * 4, work = (size_t)args.const_bytes + 1024 * CT * W;
+    return launch_kernel(rows_gemm_kernel<PL, MT, CT, W>, grid, dim3(64 * W), sums > work ? sums : work, stream,
+                         nullptr, stop, args);
+}
+template <int PL, int MT>
+hipError_t launch_tiles(const RowsArgs& args, const RowsPlan& pl, hipStream_t stream, hipEvent_t stop) {
+    if (pl.waves == 4)
+        return pl.cols == 1 ? launch_shape<PL, MT, 1, 4>(args, pl, stream, stop)
+                            : launch_shape<PL, MT, 2, 4>(args, pl, stream, stop);
+    return pl.cols == 1 ? launch_shape<PL, MT, 1, 8>(args, pl, stream, stop)
+                        : launch_shape<PL, MT, 2, 8>(args, pl, stream, stop);
+}
+template <int PL>
+hipError_t launch_planes(const RowsArgs& args, const RowsPlan& pl, hipStream_t stream, hipEvent_t stop) {
+    switch (pl.tiles) {
+        case 2: return launch_tiles<PL, 2>(args, pl, stream, stop);
+        case 3: return launch_tiles<PL, 3>(args, pl, stream, stop);
+        case 4: return launch_tiles<PL, 4>(args, pl, stream, stop);
+        default: break;
+    }
+    if constexpr (PL == 1) {
+        if (pl.tiles == 6) return launch_tiles<PL, 6>(args, pl, stream, stop);
+        if (pl.tiles == 8) return launch_tiles<PL, 8>(args, pl, stream, stop);
+    }
+    return hipErrorInvalidValue;
+}
+template <int XK>
+hipError_t launch_stage(const LinearProblem& p, u32x4* staged, float* rowscale, hipStream_t stream, hipEvent_t start) {
+    const int k = (int)p.in_features;
+    const dim3 grid((unsigned)p.rows);
+    return k <= 4096 ? launch_kernel(rows_stage_kernel<XK, 256>, grid, dim3(256), 0, stream, start, nullptr, p.x, staged, rowscale, k)
+                     : launch_kernel(rows_stage_kernel<XK, 1024>, grid, dim3(1024), 0, stream, start, nullptr, p.x, staged, rowscale, k);
+}
+}  // namespace
+
+hipError_t launch_rows(const LinearProblem& p, const RowsPlan& pl, void* workspace, hipStream_t stream,
+                       hipEvent_t start, hipEvent_t stop) {
+    u32x4* staged = (u32x4*)((char*)workspace + pl.staged_offset);
+    float* rowscale = (float*)((char*)workspace + pl.rowscale_offset);
+    const bool two = two_planes(p.x_kind);
+    RowsArgs args{};
+    args.x = (const uint16_t*)staged;
+    args.rowscale = rowscale;
+    args.qweight = p.qweight;
+    args.scales = p.scales;
+    args.zeros = p.zeros;
+    args.bias = p.bias;
+    args.bias_kind = p.bias_kind;
+    args.y = p.y;
+    args.out_kind = two ? (int)kF32 : p.x_kind;
+    args.partials = pl.splits > 1 ? (float*)workspace : nullptr;
+    args.M = (int)p.rows;
+    args.N = (int)p.out_features;
+    args.G = (int)(p.in_features / 64);
+    args.gps = pl.gps;
+    args.vec_out = (((uintptr_t)p.y & 15) == 0) && p.out_features % 4 == 0;
+    hipError_t err;
+    switch (p.x_kind) {
+        case kF16: err = launch_stage<kF16>(p, staged, rowscale, stream, start); break;
+        case kBF16: err = launch_stage<kBF16>(p, staged, rowscale, stream, start); break;
+        case kSwiGLU:
+            err = launch_kernel(rows_stage_swiglu_kernel, dim3((unsigned)p.rows, (unsigned)((p.in_features / 8 + 255) / 256)),
+                                dim3(256), 0, stream, start, nullptr, p.x, staged, rowscale, (int)p.in_features);
+            break;
+        default: err = launch_stage<kF32>(p, staged, rowscale, stream, start); break;
+    }
+    if (err != hipSuccess) return err;
+    const bool reduce = pl.splits > 1;
+    hipEvent_t gstop = reduce ? nullptr : stop;
+    err = two ? launch_planes<2>(args, pl, stream, gstop) : launch_planes<1>(args, pl, stream, gstop);
+    if (err != hipSuccess || !reduce) return err;
+    return launch_split_reduce(args.partials, p.bias, p.bias_kind, p.y, args.M, args.N, pl.splits, false, args.out_kind, stream, stop);
+}
+
+}  // namespace w4g64

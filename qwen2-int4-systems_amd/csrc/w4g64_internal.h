@@ -196,9 +196,26 @@ hipError_t launch_gemv_pipe(const LinearProblem& p, const GemvPlan& plan, void* 
 // live at the start of the workspace and a third kernel adds them up.
 bool gemm_supported(const LinearProblem& p);
 int64_t gemm_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int x_kind);
+// What launch_gemm must be given at least (the query above may answer more).
+int64_t gemm_least_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int x_kind);
 const char* gemm_kernel_name(int64_t rows, int64_t out_features, int64_t in_features, int x_kind);
-hipError_t launch_gemm(const LinearProblem& p, void* workspace, hipStream_t stream, hipEvent_t start = nullptr,
-                       hipEvent_t stop = nullptr);
+hipError_t launch_gemm(const LinearProblem& p, void* workspace, int64_t workspace_bytes, hipStream_t stream,
+                       hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
+
+// GEMM of a few row tiles (w4g64_gemm_rows.hip): 17 to 128 rows, fp32-class
+// kinds to 64.  Workspace: [split-K partial sums][staged rows][row factors].
+struct RowsPlan {
+    bool taken;  // false: the prefill GEMM
+    int tiles;   // 16-row tiles
+    int cols;    // 16-feature column tiles per workgroup
+    int waves;   // waves per workgroup
+    int splits;  // K ranges
+    int gps;     // groups per K range
+    int64_t staged_offset, rowscale_offset, workspace_bytes;
+};
+RowsPlan plan_rows(int64_t rows, int64_t out_features, int64_t in_features, int x_kind);
+hipError_t launch_rows(const LinearProblem& p, const RowsPlan& plan, void* workspace, hipStream_t stream,
+                       hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 
 // Launch a kernel; with events, hipExtLaunchKernelGGL records them at the
 // kernel's own start and end (what a profiler reports as its duration).

@@ -11,6 +11,7 @@ dequantized weights, which is checked bit for bit.
 
 from __future__ import annotations
 
+import ctypes
 import functools
 
 import numpy as np
@@ -502,6 +503,74 @@ def test_ragged_shapes(rows, n, k, dtype):
     x = O.activations(rows, k, seed=rows + n, dtype=dtype)
     bias = O._from_f32(np.linspace(-0.3, 0.3, n, dtype=np.float32), "fp16")
     check_linear(x, q, s, z, bias, n, k, dtype, bias_dtype="fp16")
+
+
+@pytest.mark.parametrize(
+    ("rows", "n", "k"),
+    [(17, 2048, 1536),    # two row tiles, the second nearly empty; eight waves
+     (33, 31, 64),        # one group: one wave has work; a ragged column tile
+     (49, 4112, 704),     # 257 column tiles (four waves), an odd group count
+     (64, 10250, 320),    # two column tiles per workgroup, the last one partial
+     (65, 130, 192),      # tiles 5 -> 6; fp32 past its limit
+     (100, 777, 8960),    # K ranges of 48 groups, the last one shorter; tiles 7 -> 8
+     (128, 96, 10304),    # 161 groups: ranges of at most 160
+     (129, 72, 512)],     # past the limit: the tiled kernel
+)
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "fp32"])
+def test_few_row_tiles(rows, n, k, dtype):
+    """The GEMM of a few row tiles at the edges of its row tiles, column tiles,
+    K ranges and waves, over a workspace left full of NaN, against the fp64
+    product of the exact weights: fp32 sums of K products of at most 15 |x|
+    carry about sqrt(K) 2^-24 of their size (and the two planes 2^-22 of x),
+    so the result is within its own rounding of the exact one plus 2^-20 of
+    the sum of magnitudes."""
+    from qwen_int4_hip import kernels
+
+    q, s, z = weights("asym", n, k, rows + n + k)
+    x = O.activations(rows, k, seed=rows + n, dtype=dtype, outliers=True)
+    bias = O._from_f32(np.linspace(-0.5, 0.5, n, dtype=np.float32), "bf16")
+    xt, (qt, st, zt), bt = to_dev(x, dtype), dev_weights(q, s, z), to_dev(bias, "bf16")
+    need = kernels._lib.load().w4g64_linear_workspace_bytes(rows, n, k, kernels._DTYPE_CODE[xt.dtype])
+    kernels._workspace(torch.device("cuda", torch.cuda.current_device()), need).fill_(0xFF)
+    got = linear_canonical_w4g64_hip(xt, qt, st, zt, bt).double()
+    w = dequantize_canonical_w4g64_hip(qt, st, zt, out_features=n, in_features=k).double()
+    exact = xt.double() @ w.t() + bt.double()
+    size = xt.double().abs() @ w.abs().t()
+    ulp = {"fp16": 2.0 ** -11, "bf16": 2.0 ** -8, "fp32": 2.0 ** -23}[dtype]
+    err = (got - exact).abs()
+    assert bool((err <= exact.abs() * ulp + size * 2.0 ** -20 + (2.0 ** -24 if dtype == "fp16" else 0.0)).all()), \
+        (err / size).max().item()
+
+
+@pytest.mark.parametrize("rows,n,k", [(17, 1536, 8960), (40, 200, 128), (64, 96, 2048)])
+def test_few_row_tiles_of_the_swiglu_product(rows, n, k):
+    """w4g64_linear_swiglu at 17..64 rows: the product staged by slices of a row
+    under a common factor (rows of very different size, a row of zeros, one
+    with an infinite gate), against fp64."""
+    from qwen_int4_hip import _lib
+
+    lib = _lib.load()
+    q, s, z = weights("asym", n, k, rows + n)
+    qt, st, zt = dev_weights(q, s, z)
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    gu = torch.randn((rows, 2 * k), generator=gen, device=DEV) * 2.0 ** torch.randint(-40, 40, (rows, 1), generator=gen,
+                                                                                     device=DEV)
+    gu[3] = 0.0
+    gu[5, k // 2] = float("inf")
+    gu = gu.to(torch.bfloat16)
+    y = torch.empty((rows, n), device=DEV)
+    need = lib.w4g64_linear_workspace_bytes(rows, n, k, _lib.DTYPE_BF16_SWIGLU)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    _lib.check(lib.w4g64_linear_swiglu(ptr(gu), ptr(qt), ptr(st), ptr(zt), None, 0, ptr(y), rows, n, k, ptr(ws), need,
+                                       ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    w = dequantize_canonical_w4g64_hip(qt, st, zt, out_features=n, in_features=k).double()
+    h = torch.nn.functional.silu(gu[:, :k].double()) * gu[:, k:].double()
+    size = h.abs() @ w.abs().t()
+    keep = torch.arange(rows, device=DEV) != 5
+    err = (y.double() - h @ w.t()).abs()
+    assert bool((err[keep] <= size[keep] * 2.0 ** -20).all()), (err[keep] / size[keep]).max().item()
+    assert bool((y[3] == 0).all()) and not bool(torch.isfinite(y[5]).any())
 
 
 @pytest.mark.parametrize(
