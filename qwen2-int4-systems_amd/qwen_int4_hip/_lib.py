@@ -99,6 +99,23 @@ def load() -> ctypes.CDLL:
     return _library
 
 
+_host_linear = None
+
+
+def host_linear():
+    """The native call of one linear (``csrc/host_linear.cpp``); raises
+    RuntimeError if it is not built."""
+    global _host_linear
+    if _host_linear is None:
+        load()
+        try:
+            from . import _host
+        except ImportError as e:
+            raise RuntimeError(f"HIP W4G64 host module is not built ({e}); run __graft_entry__.build()") from e
+        _host_linear = _host.linear
+    return _host_linear
+
+
 def check(status: int) -> None:
     """Raise the reference's exception type for a non-zero C status."""
     if status == STATUS_OK:

@@ -22,7 +22,8 @@ from __future__ import annotations
 
 import torch
 
-from .kernels import hip_available, linear_canonical_w4g64_hip
+from . import _lib
+from .kernels import _workspaces, grow_current_workspace, hip_available, linear_canonical_w4g64_hip
 from .quantization import PackingFormat, dequantize_groupwise, unpack_int4
 
 SUPPORTED_BACKENDS = ("torch", "lpu", "triton", "hip")
@@ -104,6 +105,17 @@ def hip_w4g64_linear(
     (backends.py:153-181): ``x`` is ``[..., in_features]`` fp16/bf16/fp32,
     the result is ``[..., out_features]`` in ``x.dtype``.
     """
+    # Plain calls (contiguous, aligned tensors of the contract's sizes and types
+    # on the current GPU) go through the native module, which makes the checks
+    # below; it answers None, having done nothing, for every other call.
+    if packing is PackingFormat.CANONICAL and group_size == 64 and isinstance(x, torch.Tensor) and x.is_cuda:
+        linear = _lib._host_linear or _lib.host_linear()
+        output = linear(x, qweight, scales, zeros, bias, out_features, in_features, _workspaces,
+                        grow_current_workspace)
+        if output is not None:
+            if type(output) is int:
+                _lib.check(output)
+            return output
     if not hip_available():
         raise RuntimeError("HIP backend requires a ROCm GPU and the built libw4g64_hip library")
     validate_canonical_w4g64_inputs(

@@ -1,7 +1,9 @@
-"""Build recipe for the in-tree HIP library ``libw4g64_hip.so`` (gfx950 only).
+"""Build recipe for the in-tree HIP library ``libw4g64_hip.so`` (gfx950 only)
+and the CPython module ``_host.so`` that calls it.
 
 Compiles every ``csrc/*.hip`` translation unit with hipcc (in parallel) and
-links them into ``qwen_int4_hip/libw4g64_hip.so``.  Always rebuilds: the
+links them into ``qwen_int4_hip/libw4g64_hip.so``; ``csrc/host_linear.cpp``
+(host code only) is compiled against torch's headers.  Always rebuilds: the
 caller (``__graft_entry__.build``) wants a fresh compile every time.
 
 ``build(timeline=True)`` compiles the same sources with ``-DW4G64_TIMELINE``
@@ -25,6 +27,7 @@ CSRC = SOURCE_ROOT / "csrc"
 REPO_ROOT = SOURCE_ROOT.parent
 LIBRARY = PACKAGE_DIR / "libw4g64_hip.so"
 TIMELINE_LIBRARY = PACKAGE_DIR / "libw4g64_hip_timeline.so"
+HOST_MODULE = PACKAGE_DIR / "_host.so"
 ARCH = "gfx950"
 
 HIPCC_FLAGS = [
@@ -63,6 +66,28 @@ def _compile(source: Path, obj: Path, extra: tuple = ()) -> None:
         print(stderr, file=sys.stderr)
 
 
+def build_host() -> Path:
+    """Compile ``_host.so`` (the library has to be built: it is linked)."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    tmp = HOST_MODULE.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-w",
+           "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{sysconfig.get_paths()['include']}", f"-I{root / 'include'}",
+           f"-I{root / 'include/torch/csrc/api/include'}", f"-I{Path(hipcc()).resolve().parents[1] / 'include'}",
+           str(CSRC / "host_linear.cpp"), "-o", str(tmp), f"-L{root / 'lib'}",
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+           f"-L{PACKAGE_DIR}", f"-l:{LIBRARY.name}", "-Wl,-rpath,$ORIGIN"]
+    result = subprocess.run(cmd, capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for host_linear.cpp:\n{result.stderr}")
+    os.replace(tmp, HOST_MODULE)
+    return HOST_MODULE
+
+
 def build(verbose: bool = True, timeline: bool = False) -> Path:
     """Compile and link the library (or its timeline build); returns its path."""
     sources = sorted(CSRC.glob("*.hip"))
@@ -82,6 +107,8 @@ def build(verbose: bool = True, timeline: bool = False) -> Path:
     if result.returncode != 0:
         raise RuntimeError(f"link failed:\n{result.stderr}")
     os.replace(tmp, target)
+    if not timeline:
+        build_host()
     if verbose:
         print(f"built {target} from {len(sources)} sources", file=sys.stderr)
     return target

@@ -95,6 +95,11 @@ def _workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     return _grow_workspace((index, stream.cuda_stream), nbytes, device, torch.cuda.is_current_stream_capturing())
 
 
+def grow_current_workspace(nbytes: int) -> torch.Tensor:
+    """The workspace of the current device and stream, for the native call."""
+    return _workspace(torch.device("cuda", torch.cuda.current_device()), nbytes)
+
+
 # ---------------------------------------------------------------------------
 # Primitives
 # ---------------------------------------------------------------------------
