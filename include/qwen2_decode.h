@@ -129,6 +129,29 @@ int qwen2_prefill_attention(const void* qkv, const void* cos, const void* sin, v
                             int64_t head_dim, int64_t max_length, float scale, void* workspace,
                             int64_t workspace_bytes, void* stream);
 
+/* Attention of `length` new positions per sequence after `past` cached ones,
+ * with a growing cache and a key mask (the cached-generation path of a
+ * left-padded batch).  total = past + length.
+ *   q bf16 [batch * length, num_heads * head_dim], k, v bf16 [batch * length,
+ *     num_kv_heads * head_dim]: the projections, row b * length + i;
+ *   cos, sin bf16 [batch * length, head_dim]: the rows' rotary factors;
+ *   past_k, past_v bf16 [batch, num_kv_heads, past, head_dim] (unused for past 0);
+ *   mask uint8 [batch, total] or NULL: a zero excludes the key for its sequence.
+ * Rotates q and k as qwen2_decode_attention does, writes new_k, new_v bf16
+ * [batch, num_kv_heads, total, head_dim] = the past followed by the rotated
+ * keys / the values (must not overlap the past), and writes
+ *   out[b * length + i, h * head_dim + d] =
+ *       bf16( softmax_t(q_{h,i} . k_t * scale) . v_t[d] ),
+ *       t <= past + i and mask[b, t] != 0,
+ * with fp32 scores, softmax and sums; a row without such a t gives zeros.
+ * head_dim == 128; q, k, v and the caches 16-byte aligned.
+ * Replaces: the rotary step, cache concatenation, masking and attention of
+ *           QwenAttention.forward (src/qwen_int4/model.py:61-122). */
+int qwen2_cached_attention(const void* q, const void* k, const void* v, const void* cos, const void* sin,
+                           const void* past_k, const void* past_v, const uint8_t* mask, void* new_k, void* new_v,
+                           void* out, int64_t batch, int64_t length, int64_t past, int64_t num_heads,
+                           int64_t num_kv_heads, int64_t head_dim, float scale, void* stream);
+
 /* out[r, i] = silu(gate) * up in fp32, gate = gate_up[r, i], up = gate_up[r, I + i]
  * (bf16 inputs, the fused gate|up projection), silu(x) = x / (1 + exp(-x)).
  * Replaces: the SwiGLU product of QwenMLP.forward (src/qwen_int4/model.py:133-136). */

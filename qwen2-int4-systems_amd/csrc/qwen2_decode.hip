@@ -754,8 +754,11 @@ int qwen2_prefill_attention(const void* qkv, const void* cos, const void* sin, v
     if (batch * length > 0x7FFFFFFF || batch * num_heads * tiles > 0x7FFFFFFF ||
         batch * length * num_kv_heads / 8 > 0x7FFFFFFE)
         return set_error(W4G64_STATUS_INVALID_VALUE, "problem too large");
-    PrefillArgs args;
-    args.qkv = (const uint16_t*)qkv;
+    PrefillArgs args{};
+    args.q = (const uint16_t*)qkv;
+    args.k = args.q + num_heads * kHeadDim;
+    args.v = args.k + num_kv_heads * kHeadDim;
+    args.q_row = args.kv_row = (num_heads + 2 * num_kv_heads) * kHeadDim;
     args.cos = (const uint16_t*)cos;
     args.sin = (const uint16_t*)sin;
     args.k_cache = (uint16_t*)k_cache;
@@ -769,6 +772,52 @@ int qwen2_prefill_attention(const void* qkv, const void* cos, const void* sin, v
     args.scale2 = fabsf(scale) * 1.4426950408889634f;
     args.query_sign = scale < 0.0f ? 0x80008000u : 0u;
     return launch_status(launch_prefill_attention(args, (hipStream_t)stream), "prefill_attention");
+}
+
+int qwen2_cached_attention(const void* q, const void* k, const void* v, const void* cos, const void* sin,
+                           const void* past_k, const void* past_v, const uint8_t* mask, void* new_k, void* new_v,
+                           void* out, int64_t batch, int64_t length, int64_t past, int64_t num_heads,
+                           int64_t num_kv_heads, int64_t head_dim, float scale, void* stream) {
+    if (batch < 0 || length < 0 || past < 0)
+        return set_error(W4G64_STATUS_INVALID_VALUE, "batch, length and past must be non-negative");
+    if (head_dim != kHeadDim)
+        return set_error(W4G64_STATUS_UNSUPPORTED, "head_dim must be %d, got %lld", kHeadDim, (long long)head_dim);
+    if (num_kv_heads <= 0 || num_heads <= 0 || num_heads % num_kv_heads != 0)
+        return set_error(W4G64_STATUS_INVALID_VALUE, "num_heads (%lld) must be a positive multiple of num_kv_heads (%lld)",
+                         (long long)num_heads, (long long)num_kv_heads);
+    if (batch == 0 || length == 0) return clear_error();
+    if (!q || !k || !v || !cos || !sin || !new_k || !new_v || !out || (past > 0 && (!past_k || !past_v)))
+        return set_error(W4G64_STATUS_INVALID_VALUE, "all tensors must be non-null device pointers");
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(new_k) || !aligned16(new_v) ||
+        !aligned16(past_k) || !aligned16(past_v))
+        return set_error(W4G64_STATUS_INVALID_VALUE, "q, k, v and the caches must be 16-byte aligned");
+    const int64_t total = past + length, tiles = (length + 31) / 32;
+    if (batch > 0x7FFFFFFF || num_heads > 0xFFFFFF || total > 0x7FFFFFDF || batch * total > (int64_t(1) << 40) ||
+        batch * num_heads * tiles > 0x7FFFFFFF || batch * total * num_kv_heads / 8 > 0x7FFFFFFE)
+        return set_error(W4G64_STATUS_INVALID_VALUE, "problem too large");
+    PrefillArgs args{};
+    args.q = (const uint16_t*)q;
+    args.k = (const uint16_t*)k;
+    args.v = (const uint16_t*)v;
+    args.q_row = num_heads * kHeadDim;
+    args.kv_row = num_kv_heads * kHeadDim;
+    args.cos = (const uint16_t*)cos;
+    args.sin = (const uint16_t*)sin;
+    args.past_k = (const uint16_t*)past_k;
+    args.past_v = (const uint16_t*)past_v;
+    args.mask = mask;
+    args.k_cache = (uint16_t*)new_k;
+    args.v_cache = (uint16_t*)new_v;
+    args.out = (uint16_t*)out;
+    args.batch = (int)batch;
+    args.length = (int)length;
+    args.past = (int)past;
+    args.heads = (int)num_heads;
+    args.kv_heads = (int)num_kv_heads;
+    args.max_len = (int)total;
+    args.scale2 = fabsf(scale) * 1.4426950408889634f;
+    args.query_sign = scale < 0.0f ? 0x80008000u : 0u;
+    return launch_status(launch_prefill_attention(args, (hipStream_t)stream), "cached_attention");
 }
 
 int qwen2_decode_prologue(const int64_t* token_ids, const void* embed, const int64_t* position, const float* inv_freq,

@@ -23,7 +23,17 @@
 // the keys loaded straight into operands (16 bytes of 16 rows per 16 lanes),
 // 42.7 with them through LDS, 41.5 with the lazy rescaling, 36.7 with the
 // queries rotated once per workgroup and three waves per SIMD.  At 512
-// positions 23.5 -> 13.9 us, 3000 140 -> 65, 4 x 750 55 -> 31, 16 8.6 -> 8.4.
+// positions 23.5 -> 13.9 us, 3000 140 -> 65, 4 x 750 55 -> 31, 16 8.6 -> 8.4;
+// with the queries in an LDS object of their own (one object shared with the
+// keys made every query read wait for the keys in flight) 2048 positions 35.3,
+// 512 12.9, 3000 60.9.
+//
+// The masked form serves the cached-generation layer (a growing cache, left
+// padding): a block's mask is one byte per lane, made a 32-bit word by a
+// ballot; blocks without an excluded key or a causal edge take no masking
+// instructions.  With the rotary step and the cache's concatenation in the
+// first launch it replaced some 30 torch launches: a layer over four prompts
+// of up to 300 tokens 401 -> 119 us, of which its four linears take 90.
 #include <math.h>
 
 #include <type_traits>
@@ -52,33 +62,50 @@ __device__ __forceinline__ void wait_lgkmcnt0() {
     asm volatile("" ::: "memory");
 }
 
-// One thread per 8 dimensions of a key or value head of a position.
+// One thread per 8 dimensions of a key or value head of a position: the cache's
+// earlier positions copied (kPast), the new keys rotated, the new values as they are.
+template <bool kPast>
 __global__ __launch_bounds__(256) void prefill_cache_kernel(PrefillArgs a, int64_t pieces) {
     const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (at >= pieces) return;
     constexpr int kPer = kAttnHeadDim / 8;
     const int d = 8 * (int)(threadIdx.x % kPer);
     const int64_t line = at / kPer;
-    const int row = (int)(line / (2 * a.kv_heads));            // b * length + i
-    const int head = (int)(line - (int64_t)row * 2 * a.kv_heads);  // key heads, then value heads
-    const int b = row / a.length;
-    const int i = row - b * a.length;
-    const uint16_t* vec = a.qkv + ((int64_t)row * (a.heads + 2 * a.kv_heads) + a.heads + head) * kAttnHeadDim;
-    const int kvh = head < a.kv_heads ? head : head - a.kv_heads;
-    const int64_t to = (((int64_t)b * a.kv_heads + kvh) * a.max_len + i) * kAttnHeadDim + d;
-    if (head < a.kv_heads)
-        *(u32x4*)(a.k_cache + to) = rope_piece(vec, a.cos + (int64_t)row * kAttnHeadDim, a.sin + (int64_t)row * kAttnHeadDim, d);
+    const int total = (kPast ? a.past : 0) + a.length;
+    const int64_t spot = line / (2 * a.kv_heads);                  // b * total + position
+    const int head = (int)(line - spot * 2 * a.kv_heads);          // key heads, then value heads
+    const int b = (int)(spot / total);
+    const int position = (int)(spot - (int64_t)b * total);
+    const bool key = head < a.kv_heads;
+    const int64_t slot = (int64_t)b * a.kv_heads + (key ? head : head - a.kv_heads);
+    const int64_t to = (slot * a.max_len + position) * kAttnHeadDim + d;
+    uint16_t* cache = key ? a.k_cache : a.v_cache;
+    if (kPast && position < a.past) {
+        const uint16_t* from = key ? a.past_k : a.past_v;
+        *(u32x4*)(cache + to) = *(const u32x4*)(from + (slot * a.past + position) * kAttnHeadDim + d);
+        return;
+    }
+    const int64_t row = (int64_t)b * a.length + position - (kPast ? a.past : 0);
+    const uint16_t* vec = (key ? a.k : a.v) + row * a.kv_row + (slot - (int64_t)b * a.kv_heads) * kAttnHeadDim;
+    if (key)
+        *(u32x4*)(cache + to) = rope_piece(vec, a.cos + row * kAttnHeadDim, a.sin + row * kAttnHeadDim, d);
     else
-        *(u32x4*)(a.v_cache + to) = *(const u32x4*)(vec + d);
+        *(u32x4*)(cache + to) = *(const u32x4*)(vec + d);
 }
 
+// kMasked: the queries follow `past` cached positions, and a key may be excluded
+// for a whole sequence (mask); a row without an allowed key gives zeros.
+template <bool kMasked>
 __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillArgs a) {
-    // the rotated queries, one block's keys per wave, and at the end (in the
-    // place of both) the results of two waves
-    __shared__ __attribute__((aligned(16))) unsigned char smem[(1 + kWaves) * kTile * 2 * kAttnHeadDim];
-    static_assert(sizeof(smem) >= 2 * kTile * kOutStride * 4, "two waves' results");
+    // the rotated queries; one block's keys per wave and at the end, in their
+    // place, the results of two waves (two objects: a read of the queries then
+    // does not wait for the next keys on their way to the other)
+    __shared__ __attribute__((aligned(16))) unsigned char queries[kTile * 2 * kAttnHeadDim];
+    __shared__ __attribute__((aligned(16))) unsigned char smem[2 * kTile * kOutStride * 4];
+    static_assert(sizeof(smem) >= kWaves * kTile * 2 * kAttnHeadDim, "a block's keys per wave");
     __shared__ float sm[2][kTile];
     __shared__ float sl[2][kTile];
+    __shared__ int sn[2][kTile];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the block loop branches on it
@@ -91,19 +118,23 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
     const int b = blockIdx.x % heads / a.heads;
     const int kvh = head / (a.heads / a.kv_heads);
     const int q0 = qt * kTile;
+    const int total = kMasked ? a.past + a.length : a.length;  // keys
+    // last block that a row of the tile attends to, and its first position
+    const int last = kMasked ? min(a.past + q0 + kTile - 1, total - 1) / kTile : qt;
+    const int base = kMasked ? a.past + q0 : q0;
     const int64_t cache = ((int64_t)b * a.kv_heads + kvh) * a.max_len * kAttnHeadDim;
     const uint16_t* kc = a.k_cache + cache;
     const uint16_t* vc = a.v_cache + cache;
     constexpr int kRowBytes = 2 * kAttnHeadDim;
 
-    unsigned char* stage = smem + (1 + wave) * kTile * kRowBytes;
+    unsigned char* stage = smem + wave * kTile * kRowBytes;
     u32x4 vf[8];
-    // keys and values of a block through a buffer over the prompt's rest (a
+    // keys and values of a block through a buffer over the rest of the keys (a
     // raw gfx9 buffer: rows past it read zeros, and are masked: key > query)
     auto rest = [&](const uint16_t* rows, int block) {
         const int t0 = block * kTile;
         return __builtin_amdgcn_make_buffer_rsrc((void*)(rows + (int64_t)t0 * kAttnHeadDim), 0,
-                                                 min(kTile, a.length - t0) * kRowBytes, 0x00020000);
+                                                 min(kTile, total - t0) * kRowBytes, 0x00020000);
     };
     // Keys go to LDS directly, a row's 16 pieces by 16 lanes (operand pieces
     // straight from memory would be 16 bytes of 16 rows per 16 lanes).  Piece
@@ -126,8 +157,16 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
         for (int e = 0; e < 8; ++e)
             vf[e] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, v_at + kRowBytes * (e % 4), 16 * kRowBytes * (e / 4), 0));
     };
+    // the block's mask, one key per lane (twice), loaded with its keys
+    const uint8_t* mask = kMasked && a.mask ? a.mask + (int64_t)b * total : nullptr;
+    auto load_mask = [&](int block) -> int {
+        const int t = block * kTile + (lane & 31);
+        return t < total ? (mask ? mask[t] : 1) : 0;
+    };
     int blk = wave;
-    if (blk <= qt) {
+    int mv = 0;
+    if (blk <= last) {
+        if constexpr (kMasked) mv = load_mask(blk);
         load_k(blk);
         load_v(blk);
     }
@@ -138,12 +177,13 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
     for (int u = 0; u < 2; ++u) {
         const int r = tid / 16 + 16 * u;
         const int64_t row = (int64_t)b * a.length + min(q0 + r, a.length - 1);
-        const u32x4 x = rope_piece(a.qkv + (row * (a.heads + 2 * a.kv_heads) + head) * kAttnHeadDim,
+        const u32x4 x = rope_piece(a.q + row * a.q_row + head * kAttnHeadDim,
                                    a.cos + row * kAttnHeadDim, a.sin + row * kAttnHeadDim, 8 * (tid % 16));
-        *(u32x4*)(smem + r * kRowBytes + 16 * ((tid % 16) ^ (r % 16))) = x ^ a.query_sign;
+        *(u32x4*)(queries + r * kRowBytes + 16 * ((tid % 16) ^ (r % 16))) = x ^ a.query_sign;
     }
     __syncthreads();
     float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f};
+    bool seen[2] = {false, false};  // kMasked: the row had an allowed key
     float4v o[8][2];
 #pragma unroll
     for (int dd = 0; dd < 8; ++dd)
@@ -155,9 +195,12 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
     auto step = [&](auto more) {
         constexpr bool kMore = decltype(more)::value;
         float s[2][8];
+        uint32_t word = 0;
         {
             // this block's keys have landed: the 8 value loads came after
+            // (the mask before the keys: its arrival is theirs too)
             wait_vmcnt8();
+            if constexpr (kMasked) word = (uint32_t)__ballot(mv != 0);
             u32x4 kf[2][4];
 #pragma unroll
             for (int m = 0; m < 2; ++m)
@@ -165,7 +208,10 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
                 for (int p = 0; p < 4; ++p)
                     kf[m][p] = *(const u32x4*)(stage + (16 * m + j) * kRowBytes + 16 * ((4 * p + q) ^ j));
             wait_lgkmcnt0();
-            if constexpr (kMore) load_k(blk + kWaves);
+            if constexpr (kMore) {
+                if constexpr (kMasked) mv = load_mask(blk + kWaves);
+                load_k(blk + kWaves);
+            }
             float4v acc[2][2];
 #pragma unroll
             for (int m = 0; m < 2; ++m)
@@ -175,7 +221,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
             for (int p = 0; p < 4; ++p) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    const u32x4 qv = *(const u32x4*)(smem + (16 * u + j) * kRowBytes + 16 * ((4 * p + q) ^ j));
+                    const u32x4 qv = *(const u32x4*)(queries + (16 * u + j) * kRowBytes + 16 * ((4 * p + q) ^ j));
 #pragma unroll
                     for (int m = 0; m < 2; ++m)
                         acc[m][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -187,7 +233,23 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
 #pragma unroll
                 for (int e = 0; e < 8; ++e) s[u][e] = acc[e / 4][u][e % 4];
         }
-        if (!kMore && blk == qt) {
+        if constexpr (kMasked) {
+            const int t0 = blk * kTile;
+            if (word != 0xFFFFFFFFu || t0 + kTile - 1 > base) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int most = base + 16 * u + j - t0;  // last key the row may attend to
+                    const uint32_t causal = most >= 31 ? 0xFFFFFFFFu : (most < 0 ? 0u : (2u << most) - 1u);
+                    const uint32_t own = (word & causal) >> (4 * q);  // bits 0..3 and 16..19: the lane's keys
+                    seen[u] = seen[u] || (word & causal) != 0;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (!((own >> (16 * (e / 4) + e % 4)) & 1)) s[u][e] = -INFINITY;
+                }
+            } else {
+                seen[0] = seen[1] = true;
+            }
+        } else if (!kMore && blk == qt) {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -208,16 +270,19 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
             const float mn = quarters_max(bm) * a.scale2;
             if (__any(mn - m_run[u] > 8.0f)) {
                 const float to = fmaxf(m_run[u], mn);
-                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - to);  // 2^-inf = 0 on the first block
+                float alpha = __builtin_amdgcn_exp2f(m_run[u] - to);  // 2^-inf = 0 on the first block
+                if (kMasked && to == -INFINITY) alpha = 1.0f;         // (another row's turn: no key here yet)
                 l_run[u] *= alpha;
 #pragma unroll
                 for (int dd = 0; dd < 8; ++dd) o[dd][u] *= alpha;
                 m_run[u] = to;
             }
+            // (a masked row may have met no key yet: 2^-inf, not -inf + inf)
+            const float ref = kMasked && m_run[u] == -INFINITY ? 0.0f : -m_run[u];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[u][2 * e], a.scale2, -m_run[u]));
-                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[u][2 * e + 1], a.scale2, -m_run[u]));
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[u][2 * e], a.scale2, ref));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[u][2 * e + 1], a.scale2, ref));
                 l_run[u] += p0 + p1;
                 ph[u][e] = pack_bf16x2(p0, p1);
                 pl[u][e] = pack_bf16x2(p0 - bf16_lo(ph[u][e]), p1 - bf16_hi(ph[u][e]));
@@ -240,12 +305,11 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
         }
         if constexpr (kMore) load_v(blk + kWaves);
     };
-    for (; blk + kWaves <= qt; blk += kWaves) step(std::true_type{});
-    if (blk <= qt) step(std::false_type{});
+    for (; blk + kWaves <= last; blk += kWaves) step(std::true_type{});
+    if (blk <= last) step(std::false_type{});
 
     // ---- the waves' results meet in LDS: waves 2 and 3 give theirs to 0 and
-    // 1, then wave 1 to wave 0, which stores the rows.  Wave 0 holds block 0,
-    // so its maximum is finite; a wave without a block adds 2^-inf = 0 ----
+    // 1, then wave 1 to wave 0, which stores the rows; a wave without a block (or an allowed key) adds 2^-inf = 0 ----
     float l_all[2] = {quarters_sum(l_run[0]), quarters_sum(l_run[1])};
     float(*so)[kTile][kOutStride] = (float(*)[kTile][kOutStride])smem;
 #pragma unroll
@@ -263,6 +327,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
                 if (q == 0) {
                     sm[wave - half][16 * u + j] = m_run[u];
                     sl[wave - half][16 * u + j] = l_all[u];
+                    sn[wave - half][16 * u + j] = seen[u];
                 }
             }
         }
@@ -276,6 +341,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
                 const float f = to == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run[u] - to);
                 const float fo = to == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - to);
                 m_run[u] = to;
+                seen[u] = seen[u] || sn[wave][16 * u + j] != 0;
                 l_all[u] = fmaf(sl[wave][16 * u + j], fo, l_all[u] * f);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
@@ -295,7 +361,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
     for (int u = 0; u < 2; ++u) {
         const int i = q0 + 16 * u + j;
         if (i >= a.length) continue;
-        const float inv = 1.0f / l_all[u];
+        const float inv = kMasked && !seen[u] ? 0.0f : 1.0f / l_all[u];
         uint16_t* out = a.out + (((int64_t)b * a.length + i) * a.heads + head) * kAttnHeadDim + 32 * q;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -310,13 +376,21 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
 }  // namespace
 
 hipError_t launch_prefill_attention(const PrefillArgs& args, hipStream_t stream) {
-    const int64_t pieces = (int64_t)args.batch * args.length * 2 * args.kv_heads * (kAttnHeadDim / 8);
-    hipLaunchKernelGGL(prefill_cache_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, stream, args, pieces);
+    const bool masked = args.mask || args.past > 0;
+    const int64_t pieces = (int64_t)args.batch * (args.past + args.length) * 2 * args.kv_heads * (kAttnHeadDim / 8);
+    const dim3 cgrid((unsigned)((pieces + 255) / 256));
+    if (args.past > 0)
+        hipLaunchKernelGGL(prefill_cache_kernel<true>, cgrid, dim3(256), 0, stream, args, pieces);
+    else
+        hipLaunchKernelGGL(prefill_cache_kernel<false>, cgrid, dim3(256), 0, stream, args, pieces);
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
     const int64_t tiles = ((int64_t)args.length + kTile - 1) / kTile;
-    hipLaunchKernelGGL(prefill_attention_kernel, dim3((unsigned)(tiles * args.batch * args.heads)), dim3(kThreads), 0,
-                       stream, args);
+    const dim3 grid((unsigned)(tiles * args.batch * args.heads));
+    if (masked)
+        hipLaunchKernelGGL(prefill_attention_kernel<true>, grid, dim3(kThreads), 0, stream, args);
+    else
+        hipLaunchKernelGGL(prefill_attention_kernel<false>, grid, dim3(kThreads), 0, stream, args);
     return hipGetLastError();
 }
 

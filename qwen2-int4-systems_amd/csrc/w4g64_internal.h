@@ -161,14 +161,22 @@ hipError_t launch_decode_split(const DecodeSplitArgs& args, int64_t batch, hipSt
 
 // Prompt attention (qwen2_prefill.hip).
 struct PrefillArgs {
-    const uint16_t* qkv;  // [batch * length][(heads + 2 kv_heads) * 128]
+    const uint16_t* q;    // projections of row b * length + i: heads x 128 at q + row q_row,
+    const uint16_t* k;    // kv_heads x 128 at k, v + row kv_row
+    const uint16_t* v;
+    int64_t q_row;
+    int64_t kv_row;
     const uint16_t* cos;  // [batch * length][128]
     const uint16_t* sin;
+    const uint16_t* past_k;  // [batch][kv_heads][past][128]: copied to the caches' first positions
+    const uint16_t* past_v;
+    const uint8_t* mask;  // [batch][past + length], zero: never attended to; null: all ones
     uint16_t* k_cache;    // [batch][kv_heads][max_len][128]
     uint16_t* v_cache;
     uint16_t* out;        // [batch * length][heads * 128]
     int batch;
     int length;
+    int past;
     int heads;
     int kv_heads;
     int max_len;

@@ -66,6 +66,7 @@ SIGNATURES = {
     "qwen2_decode_attention_partials": (_int, [_p] * 6 + [_i64] * 5 + [ctypes.c_float, _p, _i64, _p]),
     "qwen2_prefill_attention_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "qwen2_prefill_attention": (_int, [_p] * 6 + [_i64] * 6 + [ctypes.c_float, _p, _i64, _p]),
+    "qwen2_cached_attention": (_int, [_p] * 11 + [_i64] * 6 + [ctypes.c_float, _p]),
     "qwen2_silu_mul": (_int, [_p, _p, _i64, _i64, _p]),
     "qwen2_lm_head_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "qwen2_lm_head": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),

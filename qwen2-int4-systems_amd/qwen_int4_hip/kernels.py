@@ -237,3 +237,46 @@ def linear_canonical_w4g64_hip(
 def linear_kernel_name(rows: int, out_features: int, in_features: int, dtype: torch.dtype) -> str:
     """Name of the kernel the linear launches for this shape (for profiles)."""
     return _lib.load().w4g64_linear_kernel_name(rows, out_features, in_features, _DTYPE_CODE[dtype]).decode()
+
+
+def cached_attention_hip(q, k, v, cos, sin, past, mask, *, num_heads: int, num_kv_heads: int):
+    """Rotary step, cache concatenation, masking and attention of
+    ``QwenAttention.forward`` (src/qwen_int4/model.py:61-122) on the HIP kernels:
+    ``q`` [B, S, H * 128], ``k``, ``v`` [B, S, KVH * 128] projections, ``cos``,
+    ``sin`` [B, S, 128], ``past`` None or (key, value) [B, KVH, P, 128], ``mask``
+    [B, P + S] (zero: excluded).  Returns the attended rows [B, S, H * 128] and
+    the new (key, value) cache.  None, with nothing done, for tensors it does
+    not take: other types or devices, another head dimension, a gradient to be
+    recorded, subclasses and modes.
+    """
+    tensors = (q, k, v, cos, sin) + (() if past is None else tuple(past))
+    device = q.device
+    if q.ndim != 3 or any(type(t) is not torch.Tensor or t.dtype is not torch.bfloat16 or t.device != device
+                          for t in tensors):
+        return None
+    if device.type != "cuda" or device.index != torch.cuda.current_device() or type(mask) is not torch.Tensor:
+        return None
+    batch, length = q.shape[:2]
+    shape = (batch, length, 128)
+    if (tuple(q.shape) != (batch, length, num_heads * 128) or tuple(k.shape) != (batch, length, num_kv_heads * 128)
+            or v.shape != k.shape or tuple(cos.shape) != shape or tuple(sin.shape) != shape or num_heads % num_kv_heads
+            or mask.device != device or not batch * length
+            or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))):
+        return None
+    length_past = 0 if past is None else past[0].shape[2]
+    total = length_past + length
+    if tuple(mask.shape) != (batch, total):
+        return None
+    # (contiguous and aligned already where the linears and this function made them)
+    q, k, v, cos, sin = (t.contiguous() for t in (q, k, v, cos, sin))
+    q, k, v = (_aligned(t, 16) for t in (q, k, v))
+    past_k, past_v = (None, None) if not length_past else (_aligned(t.contiguous(), 16) for t in past)
+    mask = mask.to(torch.bool).contiguous()
+    new_k = torch.empty((batch, num_kv_heads, total, 128), dtype=torch.bfloat16, device=device)
+    new_v = torch.empty_like(new_k)
+    out = torch.empty((batch, length, num_heads * 128), dtype=torch.bfloat16, device=device)
+    lib = _require_library()
+    _lib.check(lib.qwen2_cached_attention(
+        *map(_ptr, (q, k, v, cos, sin, past_k, past_v, mask, new_k, new_v, out)), batch, length, length_past, num_heads,
+        num_kv_heads, 128, ctypes.c_float(128 ** -0.5), _stream_handle(device)))
+    return out, (new_k, new_v)

@@ -9,7 +9,10 @@ projection (:133-136) and tied bf16 LM head (:217-218).
 Attention scores are computed in fp32 (q k^T, softmax, p v) from the bf16
 q/k/v -- the reference calls scaled_dot_product_attention on bf16 tensors;
 fp32 is at least as accurate, and it keeps bf16 batched products with
-transposed operands out of the path.
+transposed operands out of the path.  With the HIP backend and heads of 128
+the rotary step, the cache's growth and the attention are two launches
+(``kernels.cached_attention_hip``); ``attend`` states the same in torch and
+serves every other case.
 
 Two cache forms:
   * ``forward(..., past_key_values, use_cache)``: the reference's growing
@@ -25,6 +28,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .kernels import cached_attention_hip
 from .linear import QuantLinear
 from .quantization import PackingFormat
 
@@ -87,27 +91,57 @@ class QwenAttention(nn.Module):
         self.o_proj = QuantLinear(self.num_heads * self.head_dim, self.hidden_size, bias=False, **common)
 
     def _project(self, hidden_states, cos, sin):
-        batch, sequence, _ = hidden_states.shape
-        q = self.q_proj(hidden_states).view(batch, sequence, self.num_heads, self.head_dim).transpose(1, 2)
-        k = self.k_proj(hidden_states).view(batch, sequence, self.num_kv_heads, self.head_dim).transpose(1, 2)
-        v = self.v_proj(hidden_states).view(batch, sequence, self.num_kv_heads, self.head_dim).transpose(1, 2)
+        return self._rotate(self.q_proj(hidden_states), self.k_proj(hidden_states), self.v_proj(hidden_states), cos, sin)
+
+    def _rotate(self, q, k, v, cos, sin):
+        batch, sequence, _ = q.shape
+        q = q.view(batch, sequence, self.num_heads, self.head_dim).transpose(1, 2)
+        k = k.view(batch, sequence, self.num_kv_heads, self.head_dim).transpose(1, 2)
+        v = v.view(batch, sequence, self.num_kv_heads, self.head_dim).transpose(1, 2)
         cos, sin = cos.unsqueeze(1), sin.unsqueeze(1)
         return q * cos + rotate_half(q) * sin, k * cos + rotate_half(k) * sin, v
+
+    def _checked_past(self, past_key_value, batch, device):
+        if past_key_value is None:
+            return None
+        past_k, past_v = past_key_value
+        expected = (batch, self.num_kv_heads, past_k.shape[2], self.head_dim)
+        if past_k.shape != expected or past_v.shape != expected:
+            raise ValueError("past key/value cache shape does not match this attention layer")
+        if past_k.device != device or past_v.device != device:
+            raise ValueError("past key/value cache must be on the attention device")
+        return past_k, past_v
+
+    def _fused(self, attention_mask) -> bool:
+        """Whether the layer may take the HIP attention: every projection on the
+        HIP backend (the others are its references), heads of 128, a key mask
+        (``QwenModel`` always passes one).  What the tensors themselves rule
+        out, ``cached_attention_hip`` answers."""
+        return (self.head_dim == 128 and attention_mask is not None and torch.cuda.is_available()
+                and all(p.backend == "hip" for p in (self.q_proj, self.k_proj, self.v_proj, self.o_proj)))
 
     def _output(self, attended, batch, sequence):
         return self.o_proj(attended.transpose(1, 2).contiguous().view(batch, sequence, self.num_heads * self.head_dim))
 
     def forward(self, hidden_states, cos, sin, attention_mask, past_key_value=None, use_cache=False):
         batch, sequence, _ = hidden_states.shape
-        q, k, v = self._project(hidden_states, cos, sin)
+        if self._fused(attention_mask):
+            projections = tuple(proj(hidden_states) for proj in (self.q_proj, self.k_proj, self.v_proj))
+            past, total = self._checked_past(past_key_value, batch, projections[1].device), sequence
+            if past is not None:
+                total += past[0].shape[2]
+            if attention_mask.shape != (batch, total):
+                raise ValueError("attention_mask must cover cached and current tokens")
+            done = cached_attention_hip(*projections, cos, sin, past, attention_mask, num_heads=self.num_heads,
+                                        num_kv_heads=self.num_kv_heads)
+            if done is not None:
+                return self.o_proj(done[0]), done[1] if use_cache else None
+            q, k, v = self._rotate(*projections, cos, sin)
+        else:
+            q, k, v = self._project(hidden_states, cos, sin)
         past_length = 0
         if past_key_value is not None:
-            past_k, past_v = past_key_value
-            expected = (batch, self.num_kv_heads, past_k.shape[2], self.head_dim)
-            if past_k.shape != expected or past_v.shape != expected:
-                raise ValueError("past key/value cache shape does not match this attention layer")
-            if past_k.device != k.device or past_v.device != v.device:
-                raise ValueError("past key/value cache must be on the attention device")
+            past_k, past_v = self._checked_past(past_key_value, batch, k.device)
             past_length = past_k.shape[2]
             k = torch.cat((past_k, k), dim=2)
             v = torch.cat((past_v, v), dim=2)

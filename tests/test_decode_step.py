@@ -449,6 +449,85 @@ def test_prefill_attention_block_edges(batch, heads, kv_heads, length, max_lengt
     assert bool((err <= bound).all()), (err - bound).max().item()
 
 
+@pytest.mark.parametrize("batch,heads,kv_heads,length,past,masking", [
+    (1, 12, 2, 1, 0, "none"),        # one row, its own key only
+    (4, 12, 2, 33, 0, "left"),       # left-padded prompts: rows without an allowed key
+    (3, 12, 2, 1, 127, "left"),      # a cached step; the new key starts a block
+    (2, 3, 3, 40, 29, "random"),     # rows cross block boundaries at an offset; any key may be excluded
+    (2, 16, 1, 65, 70, "random"),    # sixteen query heads per key/value head
+    (1, 4, 2, 300, 500, "none"),     # many blocks per wave
+    (2, 4, 4, 5, 31, "all"),         # every key excluded for one sequence
+])
+def test_cached_attention_matches_torch(batch, heads, kv_heads, length, past, masking):
+    """qwen2_cached_attention against the module path's torch restatement in
+    fp64 (bound as in the prompt attention's edge test); the cache is the
+    past followed by the rotated keys and the values, bit for bit."""
+    from qwen_int4_hip.kernels import cached_attention_hip
+
+    g = _gen(batch * 1000 + length + past)
+    d, total = 128, past + length
+    q = torch.randn((batch, length, heads * d), generator=g, device="cuda").to(torch.bfloat16)
+    k, v = (torch.randn((batch, length, kv_heads * d), generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    cache = None
+    if past:
+        cache = tuple(torch.randn((2, batch, kv_heads, past, d), generator=g, device="cuda").to(torch.bfloat16))
+    mask = torch.ones((batch, total), dtype=torch.bool, device="cuda")
+    if masking == "left":
+        for b in range(1, batch):
+            mask[b, : total * b // (batch + 1)] = False
+    elif masking == "random":
+        mask = torch.rand((batch, total), generator=g, device="cuda") < 0.7
+    elif masking == "all":
+        mask[-1] = False
+    positions = (mask.long().cumsum(-1) - 1).clamp_min(0)[:, -length:]
+    cos, sin = RotaryEmbedding(d, 1_000_000.0).cuda()(positions, torch.bfloat16)
+    out, (new_k, new_v) = cached_attention_hip(q, k, v, cos, sin, cache, mask, num_heads=heads, num_kv_heads=kv_heads)
+
+    def split(t):
+        return t.view(batch, length, -1, d).transpose(1, 2)
+
+    c, s = cos.unsqueeze(1), sin.unsqueeze(1)
+    qr = split(q) * c + rotate_half(split(q)) * s
+    kr = split(k) * c + rotate_half(split(k)) * s
+    want_k, want_v = (kr, split(v)) if cache is None else (torch.cat((cache[0], kr), 2), torch.cat((cache[1], split(v)), 2))
+    assert torch.equal(new_k, want_k) and torch.equal(new_v, want_v)
+    assert new_k.is_contiguous() and new_v.is_contiguous()
+    allowed = torch.ones((length, total), dtype=torch.bool, device="cuda").tril(past) & mask[:, None, None, :]
+    kk, vv = (t.double().repeat_interleave(heads // kv_heads, dim=1) for t in (want_k, want_v))
+    scores = torch.matmul(qr.double(), kk.transpose(-1, -2).contiguous()) * d ** -0.5
+    probs = torch.softmax(scores.masked_fill(~allowed, float("-inf")), dim=-1)
+    probs = torch.where(allowed.any(-1, keepdim=True), probs, torch.zeros_like(probs))
+    want = torch.matmul(probs, vv).transpose(1, 2).reshape(batch, length, heads * d)
+    err = (out.double() - want).abs()
+    bound = want.abs() * 2.0 ** -8 + want.abs().max() * 2.0 ** -16 * (1 + scores.abs().max())
+    assert bool((err <= bound).all()), (err - bound).max().item()
+    blind = ~allowed.any(-1).expand(batch, 1, length).squeeze(1)
+    assert bool((out[blind] == 0).all())
+
+
+def test_cached_attention_leaves_other_tensors_to_torch():
+    from qwen_int4_hip.kernels import cached_attention_hip
+
+    q = torch.randn((2, 3, 256), device="cuda").to(torch.bfloat16)
+    cos = torch.ones((2, 3, 128), device="cuda", dtype=torch.bfloat16)
+    mask = torch.ones((2, 3), device="cuda", dtype=torch.bool)
+    base = dict(q=q, k=q, v=q, cos=cos, sin=cos, past=None, mask=mask)
+    past = (torch.zeros((2, 2, 4, 128), device="cuda", dtype=torch.bfloat16),) * 2
+
+    def call(**other):
+        return cached_attention_hip(**{**base, **other}, num_heads=2, num_kv_heads=2)
+
+    assert call() is not None
+    for name, other in {"fp16": dict(q=q.half()), "host": dict(k=q.cpu()), "mask": dict(mask=mask[:, :2]),
+                        "uncovered past": dict(past=past), "head": dict(cos=cos[..., :64]),
+                        "gradient": dict(past=(past[0].clone().requires_grad_(), past[1]),
+                                         mask=torch.ones((2, 7), device="cuda", dtype=torch.bool))}.items():
+        assert call(**other) is None, name
+    strided = q.repeat(1, 1, 2)[..., :256]
+    got, want = call(q=strided, mask=mask.to(torch.int64)), call()
+    assert torch.equal(got[0], want[0])
+
+
 @pytest.mark.parametrize("rows,inter", [(1, 8960), (4, 8960), (16, 100)])
 def test_silu_mul_matches_torch(rows, inter):
     lib = _lib.load()
