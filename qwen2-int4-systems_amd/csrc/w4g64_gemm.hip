@@ -22,9 +22,8 @@
 //     keep it to 2^-40 of that magnitude.  fp32 activations (and the SwiGLU
 //     product silu(gate) * up of the down projection) become two fp16
 //     planes, hi = RNE(t) and lo = RNE(t - hi), t = x 2^-e (22 significant
-//     bits), laid out as one row [hi | lo] of 2K values; the GEMM runs over
-//     K' = 2K with weight group g mod G, so both planes meet the same
-//     weights.  fp16 activations are copied unscaled.
+//     bits), laid out as one row [hi | lo] of 2K values; both planes meet the
+//     same decoded weights in one D_g.  fp16 activations are copied unscaled.
 //   * The staging kernel also permutes each 8-value chunk into the slot
 //     order [k0 k4 k1 k5 k2 k6 k3 k7], the order in which one packed dword's
 //     nibble pairs fall out of a mask (bytes b and b + 2 share a 16-bit
@@ -53,6 +52,8 @@
 //   * Tiles are assigned so that the workgroups of one XCD (ids congruent
 //     mod 8) cover consecutive tiles of one row band: they share the
 //     activation band in their L2.
+#include <type_traits>
+
 #include "w4g64_internal.h"
 #include "w4g64_gemm.h"
 
@@ -76,8 +77,8 @@ struct GemmArgs {
     int M;
     int N;
     int K;   // staged row length (2 in_features for two planes)
-    int G;   // staged groups, K / 64
-    int wg;  // weight groups (in_features / 64): step g reads weight group g mod wg
+    int G;   // staged groups, K / 64: K steps
+    int wg;  // weight groups (in_features / 64)
     int tiles_m;
     int tiles_n;
     int band_group;  // row bands per group of the tile order (tile_coords)
@@ -156,6 +157,10 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
     constexpr int kStageBytes = kABytes + kWBytes + kSBytes + kZBytes;
     constexpr int kDma = kABytes / 1024 / NWV;  // 1 KB activation DMA instructions per wave
     constexpr int kOpsPerStep = kDma + WB + 1 + 1;  // + weight blocks, scales, zeros
+    // fp32-class rows come as two planes (and fp32 outputs come of no others):
+    // two steps per weight group, 64 rows of both planes each
+    constexpr bool kTwo = OUTK == kF32;
+    constexpr int kHalf = kBM / 2;
     __shared__ __attribute__((aligned(1024))) unsigned char smem[kStages][kStageBytes];
 
     const int tid = threadIdx.x;
@@ -210,14 +215,18 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
     // cost no vector instructions.  The host keeps the staged rows and the
     // packed weights below 2^31 elements, so the byte offsets fit 32 bits.
     // activations: instruction d writes tile rows [8 (wave kDma + d), +8), 16 B per lane
+    // Two planes: stage row r is row r % 64 of the step's half, plane r / 64;
+    // the second half is 64 rows further, where rows past M lie past the
+    // buffer's end (the offset may also wrap to one inside it).
     uint32_t a_off[kDma];
 #pragma unroll
     for (int d = 0; d < kDma; ++d) {
         const int r = 8 * (wave * kDma + d) + (lane >> 3);
         const int chunk = (lane & 7) ^ a_swizzle(r);
-        int m = (int)m0 + r;
+        int m = (int)m0 + (kTwo ? r % kHalf : r);
         m = m < a.M ? m : a.M - 1;  // rows past M load a valid row; their outputs are not stored
-        a_off[d] = 2u * ((uint32_t)m * (uint32_t)a.K + 8u * (uint32_t)chunk);
+        a_off[d] = 2u * ((uint32_t)m * (uint32_t)a.K + 8u * (uint32_t)chunk) +
+                   (kTwo && r >= kHalf ? (uint32_t)a.K : 0u);
     }
     // weights: DMA instruction b, lane L -> column nw + 32 b + L % 32, bytes [16 (L / 32), +16)
     const int c = lane & 15;   // this lane's column within a 16-column block / row within a 16-row block
@@ -236,11 +245,8 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
     const uint32_t s_row = (uint32_t)ncol * (uint32_t)a.wg;  // scale / zero element of weight group 0
     const uint32_t s_off = 2u * s_row;
     const uint32_t z_off_even = s_row >> 1, z_off_odd = (s_row >> 1) + (s_row & 1u);
-    // weight group of this workgroup's K step gg (one wrap at most: K' <= 2 in_features)
-    auto wgroup = [&](int gg) {
-        const int gabs = gbeg + gg;
-        return gabs >= a.wg ? gabs - a.wg : gabs;
-    };
+    // weight group of this workgroup's K step gg
+    auto wgroup = [&](int gg) { return kTwo ? (gbeg + gg) >> 1 : gbeg + gg; };
 
     // Buffer resources over the four operands (raw, stride 0, exact byte
     // sizes): a load's address is the per-lane offset plus a per-step scalar
@@ -253,14 +259,16 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
         __builtin_amdgcn_make_buffer_rsrc((void*)a.scales, 0, (int)((uint32_t)a.N * (uint32_t)a.wg * 2u), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t z_rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.zeros, 0, (int)(((uint32_t)a.N * (uint32_t)a.wg + 1u) >> 1), kRsrcWord3);
-    auto issue = [&](int gg) {  // callers pass gg < G only
+    auto issue = [&](int gg, auto odd) {  // callers pass gg < G only, odd: gg % 2 (two planes; else 0)
+        constexpr int kOdd = decltype(odd)::value;
         unsigned char* st = smem[gg % kStages];
         const int gw = wgroup(gg);
         const uint32_t z_off = (gw & 1) ? z_off_odd : z_off_even;
 #pragma unroll
         for (int d = 0; d < kDma; ++d)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (lds_ptr_t)(st + 1024 * (wave * kDma + d)), 16, a_off[d],
-                                                     128 * (gbeg + gg), 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rsrc, (lds_ptr_t)(st + 1024 * (wave * kDma + d)), 16,
+                                                     a_off[d] + (kOdd ? 2u * kHalf * (uint32_t)a.K : 0u), 128 * gw, 0, 0);
+        if constexpr (kOdd) return;  // the group's weights stay decoded from its first step
 #pragma unroll
         for (int bj = 0; bj < WB; ++bj)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr_t)(st + kABytes + 1024 * (WB * wave + bj)), 16,
@@ -345,12 +353,15 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
     // step g + 1.
     // "Step s has landed" for this wave = its vector memory counter is at most
     // the number of operations issued after step s's (in-order completion).
-    const int G = gcnt;  // steps of this workgroup's K range
-    issue(0);
-    if (G > 1) issue(1);
-    if (G > 2) issue(2);
-    if (G > 2) wait_vmcnt<2 * kOpsPerStep>();
-    else if (G > 1) wait_vmcnt<kOpsPerStep>();
+    constexpr std::integral_constant<int, 0> kEven{};
+    constexpr std::integral_constant<int, kTwo ? 1 : 0> kNext{};  // odd steps
+    constexpr int kOpsNext = kTwo ? kDma : kOpsPerStep;
+    const int G = gcnt;  // steps of this workgroup's K range (two planes: even)
+    issue(0, kEven);
+    if (G > 1) issue(1, kNext);
+    if (G > 2) issue(2, kEven);
+    if (G > 2) wait_vmcnt<kOpsNext + kOpsPerStep>();
+    else if (G > 1) wait_vmcnt<kOpsNext>();
     else wait_vmcnt<0>();
     block_barrier();
 
@@ -362,7 +373,80 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
 #pragma unroll
     for (int bj = 0; bj < CB; ++bj) rb[bj] = read_b(0, bj);
 
-    for (int g = 0; g < G; ++g) {
+    if constexpr (kTwo) {
+        // Both planes of a row block meet the same decoded weights in one sum
+        // per group, lo before hi (the sum is of hi's size for two products
+        // only).  Taken one after the other, as a K range of 2 K, the planes
+        // cost twice the decodes and twice the scaling, which bound the
+        // kernel: 333 x 1536x8960 fp32 47.3 -> 42.4 us per call, all launches.
+        // Step g = (group g / 2, rows 64 (g % 2) + [0, 64)); its weights are
+        // decoded in the even step.  240 -> 256 registers, no spills: B is
+        // read at the end of the odd step alone, after its scaling.
+        constexpr int HB = RB / 2;
+        u32x4 f[CB][2];
+        float sc[CB];
+        auto step = [&](int g, auto odd) {
+            constexpr int kOdd = decltype(odd)::value;
+            const unsigned char* st = smem[g % kStages];
+            // fragments (lo, hi x MFMA) of a row block, each replaced by the next
+            // row block's as soon as its products have been issued
+            u32x4 ab[4];
+#pragma unroll
+            for (int p = 0; p < 4; ++p) ab[p] = read_a(st, HB * (1 - (p >> 1)), p & 1);
+            float4v dd[2][CB];
+            auto scale_add = [&](int i) {
+                float4v(&to)[CB] = acc[HB * kOdd + i];
+#pragma unroll
+                for (int bj = 0; bj < CB; ++bj)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) to[bj][e] = __builtin_fmaf(sc[bj], dd[i & 1][bj][e], to[bj][e]);
+#pragma unroll
+                for (int bj = 0; bj < CB; ++bj) asm volatile("" : "+v"(to[bj]));
+            };
+            const int zsh = (wgroup(g) & 1) ? zsh_odd : zsh_even;
+#pragma unroll
+            for (int i = 0; i < HB; ++i) {
+                if (i + 1 == HB) {
+                    if (g + 2 < G) wait_vmcnt<kOdd ? kOpsNext : kOpsPerStep>();
+                    else wait_vmcnt<0>();
+                    if (g + 1 < G) {
+                        wait_lgkmcnt0();
+                        block_barrier();
+                        if (g + 3 < G) issue(g + 3, std::integral_constant<int, 1 - kOdd>{});
+                    }
+                }
+                float4v(&d)[CB] = dd[i & 1];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+#pragma unroll
+                    for (int bj = 0; bj < CB; ++bj) {
+                        if (!kOdd && i == 0 && p == 0) {
+                            const BConst k = group_const(zsh, rb[bj]);
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) f[bj][h] = decode_codes(rb[bj].w[h], k.zlo, k.zhi);
+                            sc[bj] = k.s;
+                        }
+                        d[bj] = mfma(ab[p], f[bj][p & 1], p == 0 ? float4v{0.f, 0.f, 0.f, 0.f} : d[bj]);
+                        if (!kOdd && i == 0 && p == 0) __builtin_amdgcn_sched_barrier(0);
+                    }
+                    if (i + 1 < HB) ab[p] = read_a(st, HB * (1 - (p >> 1)) + i + 1, p & 1);
+                }
+                if (i > 0) scale_add(i - 1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            scale_add(HB - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if (kOdd && g + 1 < G) {
+#pragma unroll
+                for (int bj = 0; bj < CB; ++bj) rb[bj] = read_b(g + 1, bj);
+            }
+        };
+        for (int g = 0; g < G; g += 2) {
+            step(g, kEven);
+            step(g + 1, kNext);
+        }
+    }
+    for (int g = 0; !kTwo && g < G; ++g) {
         const unsigned char* st = smem[g % kStages];
         u32x4 f[CB][2];  // (code - zero) of the column blocks, both MFMAs of the group
         float sc[CB];    // the column scales
@@ -415,7 +499,7 @@ __device__ __forceinline__ void gemm_body(const GemmArgs& a) {
                 if (g + 1 < G) {
                     wait_lgkmcnt0();
                     block_barrier();
-                    if (g + 3 < G) issue(g + 3);
+                    if (g + 3 < G) issue(g + 3, kEven);
                 }
             }
             float4v(&d)[CB] = dd[bi & 1];
@@ -798,6 +882,14 @@ GemmLayout gemm_layout(int64_t rows, int64_t out_features, int64_t in_features, 
     l.staged_offset = up256(l.plan.partial_bytes);
     l.rowscale_offset = l.staged_offset + up256(rows * k_staged * 2);
     l.bytes = l.rowscale_offset + padded_rows * 4;
+    if (two_planes(x_kind) && l.plan.split_tiles && l.plan.gps % 2) {  // K ranges of whole groups: two steps each
+        l.plan.gps += 1;
+        l.plan.splits = (int)((k_staged / 64 + l.plan.gps - 1) / l.plan.gps);
+        if (l.plan.splits == 1) {  // (one group in two ranges)
+            l.plan.dp_tiles += l.plan.split_tiles;
+            l.plan.split_tiles = 0;
+        }
+    }
     return l;
 }
 

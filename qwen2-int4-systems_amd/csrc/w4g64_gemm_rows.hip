@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64 * W) void rows_gemm_kernel(RowsArgs a) {
             for (int c = 0; c < CT; ++c) {
                 float4v d = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int p = 0; p < PL; ++p)
+                for (int p = PL - 1; p >= 0; --p)  // lo before hi: the sum is of hi's size for two products only
 #pragma unroll
                     for (int h = 0; h < 2; ++h)
                         d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, t.x[m][p][h]),

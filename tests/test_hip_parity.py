@@ -575,6 +575,26 @@ def test_few_row_tiles_of_the_swiglu_product(rows, n, k):
 
 @pytest.mark.parametrize(
     ("rows", "n", "k"),
+    [(65, 72, 64),        # one group: two steps; the second half holds one row
+     (128, 130, 192),     # a full tile
+     (129, 300, 320),     # the last tile's second half empty
+     (200, 264, 4160),    # 65 groups in K ranges of whole groups
+     (333, 1536, 8960),   # the module path's down projection
+     (600, 28000, 192)],  # more tiles than workgroup slots: whole and split ones
+)
+def test_two_planes_in_one_sum(rows, n, k):
+    """fp32 rows of the 128 x 256 tiles: both planes of a group in one sum, at
+    the edges of the row halves, K ranges and tiles (bound as above)."""
+    test_few_row_tiles(rows, n, k, "fp32")
+
+
+@pytest.mark.parametrize("rows,n,k", [(70, 72, 64), (160, 520, 1984)])
+def test_two_planes_of_the_swiglu_product(rows, n, k):
+    test_few_row_tiles_of_the_swiglu_product(rows, n, k)
+
+
+@pytest.mark.parametrize(
+    ("rows", "n", "k"),
     [(9, 1536, 1536), (12, 256, 1536), (16, 8960, 1536), (16, 1536, 8960), (13, 72, 3072), (16, 40, 9280),
      (10, 96, 64), (9, 8200, 512), (12, 7, 192), (16, 13, 8960)],
 )
