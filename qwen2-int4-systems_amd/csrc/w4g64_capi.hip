@@ -17,7 +17,7 @@
 #include "w4g64_internal.h"
 
 // The allocation-free entry point's scratch (w4g64_linear_static_scratch).
-constexpr int64_t kScratchBytes = 4ll << 20;
+using w4g64::kScratchBytes;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {

@@ -893,13 +893,14 @@ GemmLayout gemm_layout(int64_t rows, int64_t out_features, int64_t in_features, 
     return l;
 }
 
-// Few row tiles have a kernel of their own, faster at every size measured up to
-// its limits (w4g64_gemm_rows.hip), where the workspace holds its plan.  The
-// tiled plan's bytes stay what a call must bring, and what the workspace query
-// answers unless the other plan needs a little more (rows padded to 32, short
-// K), so that no caller's scratch (w4g64_linear_static_scratch among them)
-// becomes too small or is suddenly large enough.
-constexpr int64_t kFewRowsExtra = 1 << 20;
+// Fewer products have a kernel of their own (w4g64_gemm_rows.hip, whose planner
+// draws the line), where the workspace holds its plan.  The tiled plan's bytes
+// stay what a call must bring, and what the workspace query answers unless the
+// other plan needs more (rows padded to whole tiles) on the same side of the
+// static scratch: what w4g64_linear_static_scratch takes and refuses stays.
+bool few_rows_fit(const RowsPlan& few, int64_t tiled) {
+    return few.taken && (few.workspace_bytes <= kScratchBytes || tiled > kScratchBytes);
+}
 
 }  // namespace
 
@@ -910,7 +911,7 @@ int64_t gemm_least_workspace_bytes(int64_t rows, int64_t out_features, int64_t i
 int64_t gemm_workspace_bytes(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
     const int64_t tiled = gemm_least_workspace_bytes(rows, out_features, in_features, x_kind);
     const RowsPlan few = plan_rows(rows, out_features, in_features, x_kind);
-    return few.taken && few.workspace_bytes > tiled && few.workspace_bytes <= kFewRowsExtra ? few.workspace_bytes : tiled;
+    return few_rows_fit(few, tiled) && few.workspace_bytes > tiled ? few.workspace_bytes : tiled;
 }
 
 bool gemm_supported(const LinearProblem& p) {
@@ -923,7 +924,7 @@ bool gemm_supported(const LinearProblem& p) {
 const char* gemm_kernel_name(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
     const GemmLayout l = gemm_layout(rows, out_features, in_features, x_kind);
     const RowsPlan few = plan_rows(rows, out_features, in_features, x_kind);
-    if (few.taken && few.workspace_bytes <= (l.bytes > kFewRowsExtra ? l.bytes : kFewRowsExtra)) {
+    if (few_rows_fit(few, l.bytes)) {
         if (x_kind == kF16) return "gemm_kernel<f16 a x int b,few rows> (fp16 rows staged)";
         if (x_kind == kBF16) return "gemm_kernel<f16 a x int b,few rows> (bf16 rows staged as scaled fp16)";
         if (x_kind == kSwiGLU) return "gemm_kernel<f16 a x int b,few rows> (silu(gate)*up staged as scaled fp16 hi|lo)";

@@ -1,5 +1,5 @@
-// W4G64 GEMM for a few row tiles (17 to 128 rows; fp32-class activations to
-// 64): batched decode, draft verification, short prompts.  The arithmetic is
+// W4G64 GEMM for few products (17 rows up to short prompts; plan_rows draws the
+// line): batched decode, draft verification, prompts of a few hundred tokens.  The arithmetic is
 // the prefill GEMM's (w4g64_gemm.hip): staged fp16 rows times a power of two,
 // exact integer (code - zero) on the matrix cores, the group scale in fp32,
 // the row factor last.  What differs is the shape: a 128 x 256 tile is mostly
@@ -11,8 +11,9 @@
 //       operand order [row tile][group][plane][half][lane][8], so that an
 //       operand load is a contiguous kilobyte.
 //   rows_gemm_kernel
-//       one workgroup of W waves per 16 CT output features and K range.  Each
-//       wave takes a contiguous part of the range's groups over all rows;
+//       one workgroup of W waves per 16 CT output features, row block of MT
+//       row tiles and K range.  Each wave takes a contiguous part of the
+//       range's groups over all of the block's rows;
 //       the waves' sums meet in LDS at the end.  Two planes meet the same
 //       decoded weights, in one sum per group.
 //
@@ -24,8 +25,9 @@
 // workgroup, 8.  Per call with the staging and any reduction, bf16,
 // graph-replayed over rotated weights, against the 128 x 256 tiles: 24 x
 // 17920x1536 29.0 -> 11.6 us, 24 x 1536x1536 16.0 -> 6.8, 40 x 8960x1536 23.1
-// -> 11.1, 128 x 8960x1536 27.9 -> 19.2, 24 x 1536x8960 of the SwiGLU
-// product (fp32) 33.2 -> 16.1, 64 x 1536x8960 fp32 32.7 -> 22.4.
+// -> 11.1, 128 x 8960x1536 27.9 -> 16.1, 512 x 1536x1536 24.7 -> 14.3, 24 x
+// 1536x8960 of the SwiGLU product (fp32) 33.2 -> 16.1, 64 x 1536x8960 fp32 32.7
+// -> 22.4.
 #include "w4g64_gemm.h"
 #include "w4g64_internal.h"
 
@@ -187,6 +189,7 @@ __global__ __launch_bounds__(64 * W) void rows_gemm_kernel(RowsArgs a) {
     const int j = lane & 15;
     const int q = lane >> 4;
     const int n0 = blockIdx.x * kCols;
+    const int t0 = blockIdx.z * MT;        // first row tile
     const int first = blockIdx.y * a.gps;  // (gps is even)
     const int count = min(a.gps, a.G - first);
     const int pairs = (count + 1) / 2;
@@ -198,7 +201,8 @@ __global__ __launch_bounds__(64 * W) void rows_gemm_kernel(RowsArgs a) {
     unsigned char* mine = smem + a.const_bytes + 1024 * CT * wave;
 
     const __amdgpu_buffer_rsrc_t x_rsrc =
-        __builtin_amdgcn_make_buffer_rsrc((void*)a.x, 0, (int)((uint32_t)(MT * a.G) * (2048u * PL)), kRsrcWord3);
+        __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + (int64_t)t0 * a.G * (1024 * PL)), 0,
+                                          (int)((uint32_t)(MT * a.G) * (2048u * PL)), kRsrcWord3);
     const __amdgpu_buffer_rsrc_t w_rsrc =
         __builtin_amdgcn_make_buffer_rsrc((void*)a.qweight, 0, (int)((uint32_t)a.N * (uint32_t)a.G * 32u), kRsrcWord3);
 
@@ -328,13 +332,14 @@ __global__ __launch_bounds__(64 * W) void rows_gemm_kernel(RowsArgs a) {
             for (int r = 0; r < 4; ++r) so[wave][16 * m + 4 * q + r][16 * c + j] = acc[m][c][r];
     __syncthreads();
     for (int e = tid; e < kRows * kCols / 4; e += 64 * W) {
-        const int row = e / (kCols / 4);
+        const int local = e / (kCols / 4);
+        const int row = 16 * t0 + local;
         const int col = 4 * (e % (kCols / 4));
         const int n = n0 + col;
         if (row >= a.M || n >= a.N) continue;
-        float4v sum = *(const float4v*)&so[0][row][col];
+        float4v sum = *(const float4v*)&so[0][local][col];
 #pragma unroll
-        for (int w = 1; w < W; ++w) sum += *(const float4v*)&so[w][row][col];
+        for (int w = 1; w < W; ++w) sum += *(const float4v*)&so[w][local][col];
         sum *= a.rowscale[row];
         const int64_t at = (int64_t)row * a.N + n;
         if (a.partials) {
@@ -365,38 +370,73 @@ bool two_planes(int x_kind) { return x_kind == kF32 || x_kind == kSwiGLU; }
 
 }  // namespace
 
-// Waves and columns per workgroup, K ranges.  Measured per call (24, 40, 64
-// and 96 rows; CT x W with one range, or with the ranges given):
+// Row blocks, waves and columns per workgroup, K ranges.  Measured per call.
+// Up to four row tiles (two of two planes with K to 4096), one block (24, 40
+// and 64 rows; CT x W with one range, or with the ranges given):
 //   up to 256 column tiles, K up to 4096: 1 x 8 (2048x1536 at 24 rows 7.0 us
 //     against 7.2 for 1 x 4 and 7.6 for 2 x 8; 4096x4096 at 40 11.0, 11.7, 12.3);
 //   more column tiles: 1 x 4 while they are few enough to be one round of
 //     workgroups (8960x1536 at 40 rows 11.1, 2 x 4 11.6; 17920x1536 at 24 12.0,
-//     2 x 4 11.6) and the rows' loads do not dominate (96 rows 16.8, 2 x 4 15.9);
+//     2 x 4 11.6);
 //   longer K: 2 x 8 and as many ranges as keep one workgroup per CU
 //     (1536x8960 at 40 rows: one range 17.0, two of 1 x 8 15.0, four of 2 x 8
 //     14.7).
+// More rows: blocks of two row tiles, 2 x 8, while those are at most one
+// workgroup per CU (128 x 1536x1536 8.0 us, blocks of four 9.4, one of eight
+// 10.1), else of up to four, with four waves past one workgroup per CU (256 x
+// 8960x1536 22.8, blocks of eight 27.0; 512 x 1536x1536 14.3, eight waves 16.9);
+// 64 x 8960x1536 of two planes 19.3 in one block, 14.0 in two.
+// The line to the 128 x 256 tiles (that kernel | this one):
+//   one round of workgroups, or K of 1024 to 4096 up to 6e9 products: 160 x
+//     1536x1536 18.9 | 9.5, 2048 x 256x1536 26.6 | 19.1, 512 x 2048x1536 27.0 |
+//     15.1, 512 x 8960x1536 37.5 | 36.1, 200 x 16384x2560 44.1 | 43.9;
+//   shorter K is the join of the waves' sums alone: 2048 x 1536x256 14.4 | 16.5;
+//   longer K: 256 x 1536x8960 32.8 | 27.0, but 512 x 1536x8960 39.5 | 40.9 and
+//     200 x 10000x6400 63.0 | 67.9;
+//   many rows of few features, where the staging decides: 4096 x 256x1536
+//     28.3 | 30.5;
+//   two planes: 512 x 4096x1536 35.1 | 30.8, 333 x 8960x1536 43.5 | 41.8, 160 x
+//     1536x8960 36.2 | 27.5, but 256 x 1536x8960 36.7 | 42.0, 512 x 512x9216
+//     35.0 | 43.8 and 2048 x 256x1536 25.7 | 30.4.
 // A range holds at most 160 groups (40 KB of scales and zero points in LDS).
 RowsPlan plan_rows(int64_t rows, int64_t out_features, int64_t in_features, int x_kind) {
     RowsPlan pl{};
     const bool two = two_planes(x_kind);
     const int64_t tiles = (rows + 15) / 16;
-    if (tiles < 2 || tiles > (two ? 4 : 8)) return pl;
-    pl.tiles = (int)(tiles == 5 ? 6 : (tiles == 7 ? 8 : tiles));
-    const int64_t staged = (int64_t)pl.tiles * 16 * in_features * (two ? 4 : 2);
-    if (staged >= (int64_t(1) << 31)) return pl;  // 32-bit operand offsets
+    if (tiles < 2) return pl;
     const int G = (int)(in_features / 64);
     const int64_t columns = (out_features + 15) / 16;
+    pl.blocks = 1;
     pl.cols = 1;
     pl.waves = 8;
     int64_t splits = 1;
-    if (G > 64) {
+    const int64_t pairs = (columns + 1) / 2;
+    if (tiles > 4 || (two && tiles > 2 && G <= 64)) {
+        const int64_t most = pairs * ((tiles + 1) / 2) <= 256 ? 2 : 4;  // tiles per block
+        const int64_t blocks = (tiles + most - 1) / most;
+        pl.tiles = (int)((tiles + blocks - 1) / blocks);
+        pl.blocks = (int)blocks;
         pl.cols = 2;
-        splits = 224 / ((columns + 1) / 2);
-        splits = splits < G / 16 ? splits : G / 16;
-    } else if (columns > 256) {
-        pl.cols = columns <= 640 && tiles <= 4 ? 1 : 2;
-        pl.waves = 4;
+        pl.waves = pairs * blocks <= 256 ? 8 : 4;
+        const double products = (double)rows * (double)out_features * (double)in_features;
+        if (tiles > (two ? 4 : 8)) {
+            if (rows > (two ? 1024 : 2048)) return pl;
+            if (G > 64 && (two ? most > 2 || products > 2.3e9 : pairs * blocks > 256 && products > 4e9)) return pl;
+            if (G <= 64 && pairs * blocks > 256 && (G < 16 || products > (two ? 4e9 : 6e9))) return pl;
+        }
+    } else {
+        pl.tiles = (int)tiles;
+        if (G > 64) {
+            pl.cols = 2;
+            splits = 224 / pairs;
+            splits = splits < G / 16 ? splits : G / 16;
+        } else if (columns > 256) {
+            pl.cols = columns <= 640 ? 1 : 2;
+            pl.waves = 4;
+        }
     }
+    const int64_t staged = (int64_t)pl.blocks * pl.tiles * 16 * in_features * (two ? 4 : 2);
+    if (staged >= (int64_t(1) << 31)) return pl;  // 32-bit operand offsets
     const int64_t least = (G + 159) / 160;
     splits = splits < least ? least : splits;
     pl.gps = (int)((G + splits - 1) / splits + 1) / 2 * 2;
@@ -413,7 +453,7 @@ namespace {
 template <int PL, int MT, int CT, int W>
 hipError_t launch_shape(RowsArgs args, const RowsPlan& pl, hipStream_t stream, hipEvent_t stop) {
     args.const_bytes = args.gps * 16 * CT * 8;
-    const dim3 grid((unsigned)((args.N + 16 * CT - 1) / (16 * CT)), (unsigned)pl.splits);
+    const dim3 grid((unsigned)((args.N + 16 * CT - 1) / (16 * CT)), (unsigned)pl.splits, (unsigned)pl.blocks);
     const size_t sums = (size_t)W * (16 * MT) * (16 * CT + 4) * 4, work = (size_t)args.const_bytes + 1024 * CT * W;
     return launch_kernel(rows_gemm_kernel<PL, MT, CT, W>, grid, dim3(64 * W), sums > work ? sums : work, stream,
                          nullptr, stop, args);
@@ -433,10 +473,6 @@ hipError_t launch_planes(const RowsArgs& args, const RowsPlan& pl, hipStream_t s
         case 3: return launch_tiles<PL, 3>(args, pl, stream, stop);
         case 4: return launch_tiles<PL, 4>(args, pl, stream, stop);
         default: break;
-    }
-    if constexpr (PL == 1) {
-        if (pl.tiles == 6) return launch_tiles<PL, 6>(args, pl, stream, stop);
-        if (pl.tiles == 8) return launch_tiles<PL, 8>(args, pl, stream, stop);
     }
     return hipErrorInvalidValue;
 }

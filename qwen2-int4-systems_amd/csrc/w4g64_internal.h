@@ -210,11 +210,15 @@ const char* gemm_kernel_name(int64_t rows, int64_t out_features, int64_t in_feat
 hipError_t launch_gemm(const LinearProblem& p, void* workspace, int64_t workspace_bytes, hipStream_t stream,
                        hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 
+// The allocation-free entry point's scratch (w4g64_linear_static_scratch).
+constexpr int64_t kScratchBytes = 4ll << 20;
+
 // GEMM of a few row tiles (w4g64_gemm_rows.hip): 17 to 128 rows, fp32-class
 // kinds to 64.  Workspace: [split-K partial sums][staged rows][row factors].
 struct RowsPlan {
     bool taken;  // false: the prefill GEMM
-    int tiles;   // 16-row tiles
+    int tiles;   // 16-row tiles per row block, 2 to 4
+    int blocks;  // row blocks
     int cols;    // 16-feature column tiles per workgroup
     int waves;   // waves per workgroup
     int splits;  // K ranges

@@ -588,7 +588,21 @@ def test_two_planes_in_one_sum(rows, n, k):
     test_few_row_tiles(rows, n, k, "fp32")
 
 
-@pytest.mark.parametrize("rows,n,k", [(70, 72, 64), (160, 520, 1984)])
+@pytest.mark.parametrize(
+    ("rows", "n", "k"),
+    [(129, 777, 704),    # blocks of two row tiles, the last one nearly empty
+     (200, 1300, 320),   # blocks of four, eight waves
+     (300, 4112, 1024),  # more than one workgroup per CU: four waves
+     (333, 40, 10304),   # 161 groups: two K ranges over row blocks
+     (1024, 48, 64),     # many row blocks of one group
+     (2048, 33, 192)],   # the most rows (two planes: the tiled kernel)
+)
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "fp32"])
+def test_row_blocks(rows, n, k, dtype):
+    test_few_row_tiles(rows, n, k, dtype)
+
+
+@pytest.mark.parametrize("rows,n,k", [(70, 72, 64), (160, 520, 1984), (260, 2600, 4160)])
 def test_two_planes_of_the_swiglu_product(rows, n, k):
     test_few_row_tiles_of_the_swiglu_product(rows, n, k)
 
