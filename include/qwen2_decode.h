@@ -177,6 +177,16 @@ int64_t qwen2_lm_head_workspace_bytes(int64_t rows, int64_t vocab, int64_t hidde
 int qwen2_lm_head(const void* x, const void* weight, void* logits, int64_t* argmax, int64_t rows, int64_t vocab,
                   int64_t hidden, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The greedy choice alone, over logits bf16 [rows, vocab] of any head:
+ * argmax[r] as qwen2_lm_head's.  rows <= 65535; argmax and workspace 8-byte
+ * aligned.  Bytes of workspace: one key per row and 4096 logits, 0 for
+ * unsupported sizes; calls sharing it must be ordered on one stream.
+ * Replaces: logits[:, -1].argmax(dim=-1) (src/qwen_int4/generation.py:51)
+ *           past qwen2_lm_head's 16 rows. */
+int64_t qwen2_argmax_workspace_bytes(int64_t rows, int64_t vocab);
+int qwen2_argmax(const void* logits, int64_t* argmax, int64_t rows, int64_t vocab, void* workspace,
+                 int64_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -70,6 +70,8 @@ SIGNATURES = {
     "qwen2_silu_mul": (_int, [_p, _p, _i64, _i64, _p]),
     "qwen2_lm_head_workspace_bytes": (_i64, [_i64, _i64, _i64]),
     "qwen2_lm_head": (_int, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _i64, _p]),
+    "qwen2_argmax_workspace_bytes": (_i64, [_i64, _i64]),
+    "qwen2_argmax": (_int, [_p, _p, _i64, _i64, _p, _i64, _p]),
 }
 
 _lock = threading.Lock()

@@ -225,6 +225,10 @@ class FusedDecodeStep:
         # the HIP LM head (with fused greedy argmax) covers up to 16 rows
         hws = self.lib.qwen2_lm_head_workspace_bytes(batch, self.vocab, self.hidden)
         self.hip_head = hws > 0 and head.dtype == bf16 and head.is_contiguous()
+        self.hip_argmax = False
+        if not self.hip_head:  # the greedy choice over torch's logits
+            hws = self.lib.qwen2_argmax_workspace_bytes(batch, self.vocab)
+            self.hip_argmax = hws > 0
         self.head_workspace = torch.zeros(max(hws, 1), dtype=torch.uint8, device=device)
 
     def _linear(self, x, code, weights, y, stream) -> None:
@@ -337,7 +341,14 @@ class FusedDecodeStep:
         if not self.hip_head:
             logits = F.linear(self.normed, model.lm_head.weight)
             if next_token is not None:
-                next_token.copy_(logits.argmax(dim=-1, keepdim=True))
+                if (self.hip_argmax and logits.dtype == torch.bfloat16 and logits.is_contiguous()
+                        and next_token.dtype == torch.int64
+                        and next_token.shape == (self.batch, 1) and next_token.is_contiguous()
+                        and next_token.device == logits.device):
+                    _lib.check(self.lib.qwen2_argmax(_ptr(logits), _ptr(next_token), self.batch, self.vocab,
+                                                     _ptr(self.head_workspace), self.head_workspace.numel(), stream))
+                else:
+                    next_token.copy_(logits.argmax(dim=-1, keepdim=True))
             return logits.view(self.batch, 1, -1)
         logits = torch.empty((self.batch, self.vocab), dtype=torch.bfloat16, device=self.device)
         if next_token is not None and (next_token.dtype != torch.int64 or next_token.numel() != self.batch

@@ -822,6 +822,28 @@ def test_lm_head_argmax_ties_and_nan():
     assert argmax[2].item() == 0 and argmax[3].item() == 0
 
 
+@pytest.mark.parametrize("rows,vocab", [(1, 1), (3, 4095), (17, 4096), (24, 4097), (5, 8200), (33, 151936)])
+def test_argmax_of_any_rows(rows, vocab):
+    """qwen2_argmax at the edges of its slices, aligned rows and not, with ties
+    over slices, NaN, infinities and zeros of both signs."""
+    lib = _lib.load()
+    logits = torch.randn((rows, vocab), generator=_gen(vocab), device="cuda").to(torch.bfloat16)
+    logits[0] = float("-inf")
+    if rows > 2:
+        logits[1, vocab // 3] = logits[1, vocab - 1] = logits[1].max() + 1  # the first of two
+        logits[2] = -0.0
+        logits[2, vocab // 2] = 0.0  # equal to -0: index 0
+    if rows > 4:
+        logits[3, vocab - 1] = float("nan")
+        logits[4, vocab - 2:] = float("inf")
+    need = lib.qwen2_argmax_workspace_bytes(rows, vocab)
+    workspace = torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda")
+    got = torch.empty(rows, dtype=torch.int64, device="cuda")
+    _lib.check(lib.qwen2_argmax(_p(logits), _p(got), rows, vocab, _p(workspace), need, _stream()))
+    assert torch.equal(got, _first_argmax(logits))
+    assert lib.qwen2_argmax(_p(logits), _p(got), rows, vocab, _p(workspace), need - 1, _stream()) != 0
+
+
 def test_lm_head_repeated_calls_share_the_workspace():
     """Back-to-back calls on one stream reuse one workspace."""
     lib = _lib.load()
