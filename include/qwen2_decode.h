@@ -104,8 +104,8 @@ int qwen2_decode_attention_partials(const void* qkv, const void* cos, const void
                                     int64_t num_kv_heads, int64_t head_dim, int64_t max_length, float scale,
                                     void* workspace, int64_t workspace_bytes, void* stream);
 
-/* Bytes of workspace qwen2_prefill_attention needs: the rotated queries,
- * bf16 [batch, num_heads, length, head_dim]. */
+/* Bytes of workspace qwen2_prefill_attention must be given: bf16 [batch,
+ * num_heads, length, head_dim] (checked, not written). */
 int64_t qwen2_prefill_attention_workspace_bytes(int64_t batch, int64_t num_heads, int64_t length);
 
 /* Attention over a prompt of `length` positions per sequence.

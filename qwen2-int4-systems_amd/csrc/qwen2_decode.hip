@@ -663,11 +663,16 @@ static int decode_attention(const void* qkv, const void* cos, const void* sin, v
     // Batch 1 with a cache of up to 1024 positions: the single kernel, whose
     // chunks and merge are those of the o_proj linear's own merge
     // (w4g64_linear_attention_merge), so the two forms agree bit for bit.  It
-    // is also as fast there (position 575 of 640: 7.9 us either way).  Past
-    // that the split kernel is the faster one at every size measured (2 x 640
-    // positions 8.1 -> 8.0 us, 24 x 1024 28.0 -> 11.7, 8 x 4096 51 -> 12.7):
-    // each chunk's arrival costs an agent-scope release.
-    if (!unmerged && (batch > 1 || chunks > kAttnMergeMaxChunks)) {
+    // is also as fast there (position 575 of 640: 7.9 us either way).  Other
+    // calls take the split kernel, whose workgroups don't pay an agent-scope
+    // release per chunk (2 x 64 positions 8.4 -> 5.5 us, 24 x 1024 28.0 -> 11.7,
+    // 8 x 4096 51 -> 12.7), except where it needs its second launch for few
+    // chunks: graph-replayed it saves 0.2 to 0.5 us there (2 x 640, two key
+    // heads, 40 chunks, 8.7 -> 8.4), but launched one by one the second launch
+    // costs 1.3 us (10.5 -> 11.8).  Past 96 chunks it is ahead either way (128:
+    // 10.3 -> 8.5 and 11.9 -> 11.7).
+    const int splits = decode_splits(batch, num_kv_heads, max_length);
+    if (!unmerged && (chunks > kAttnMergeMaxChunks || (batch > 1 && (splits == 1 || blocks > 96)))) {
         DecodeSplitArgs sp;
         sp.qkv = (const uint16_t*)qkv;
         sp.cos = (const uint16_t*)cos;
@@ -680,7 +685,7 @@ static int decode_attention(const void* qkv, const void* cos, const void* sin, v
         sp.heads = (int)num_heads;
         sp.kv_heads = (int)num_kv_heads;
         sp.max_len = (int)max_length;
-        sp.splits = decode_splits(batch, num_kv_heads, max_length);
+        sp.splits = splits;
         sp.scale2 = scale * 1.4426950408889634f;
         return launch_status(launch_decode_split(sp, batch, (hipStream_t)stream), "decode_attention");
     }

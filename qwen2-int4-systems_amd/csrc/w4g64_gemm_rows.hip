@@ -389,7 +389,8 @@ bool two_planes(int x_kind) { return x_kind == kF32 || x_kind == kSwiGLU; }
 // The line to the 128 x 256 tiles (that kernel | this one):
 //   one round of workgroups, or K of 1024 to 4096 up to 6e9 products: 160 x
 //     1536x1536 18.9 | 9.5, 2048 x 256x1536 26.6 | 19.1, 512 x 2048x1536 27.0 |
-//     15.1, 512 x 8960x1536 37.5 | 36.1, 200 x 16384x2560 44.1 | 43.9;
+//     15.1, 333 x 8960x1536 35.9 | 28.7, 2048 x 1536x1536 40.6 | 33.3; past
+//     that they meet: 512 x 8960x1536 37.5 | 36.1, 200 x 16384x2560 44.1 | 43.9;
 //   shorter K is the join of the waves' sums alone: 2048 x 1536x256 14.4 | 16.5;
 //   longer K: 256 x 1536x8960 32.8 | 27.0, but 512 x 1536x8960 39.5 | 40.9 and
 //     200 x 10000x6400 63.0 | 67.9;

@@ -179,6 +179,9 @@ def test_decode_attention_matches_torch(batch, heads, kv_heads, max_length, posi
     (33, 14, 2, 300, (0, 200, 299)),                # seven per head; fewer splits than the cache has room for
     (1, 16, 2, 17408, (31, 4095, 17407)),           # the longest cache, the most splits
     (2, 12, 2, 640, (-5, 640, 10_000)),             # clamped to the cache
+    (24, 16, 2, 129, (0, 127, 128)),                # past 96 chunks: two splits of the split kernel
+    (3, 3, 3, 1000, (3, 126, 511, 512, 999)),
+    (6, 12, 2, 640, (-5, 640, 10_000)),
 ])
 def test_decode_attention_split_over_workgroups(batch, heads, kv_heads, max_length, positions):
     """qwen2_decode_attention past one sequence or 1024 positions (the split
