@@ -26,7 +26,7 @@
 // graph-replayed over rotated weights, against the 128 x 256 tiles: 24 x
 // 17920x1536 29.0 -> 11.6 us, 24 x 1536x1536 16.0 -> 6.8, 40 x 8960x1536 23.1
 // -> 11.1, 128 x 8960x1536 27.9 -> 16.1, 512 x 1536x1536 24.7 -> 14.3, 24 x
-// 1536x8960 of the SwiGLU product (fp32) 33.2 -> 16.1, 64 x 1536x8960 fp32 32.7
+// 1536x8960 of the SwiGLU product (fp32) 33.2 -> 16.6, 64 x 1536x8960 fp32 32.7
 // -> 22.4.
 #include "w4g64_gemm.h"
 #include "w4g64_internal.h"
@@ -125,50 +125,44 @@ __global__ __launch_bounds__(THREADS) void rows_stage_kernel(const void* x, u32x
 
 // The SwiGLU product, one workgroup per row and 2048 values: its exponentials
 // and divisions, on one CU per row, took 7.0 us at 24 x 8960.  Every
-// workgroup of a row scans all of it for the largest finite |gate| and |up|,
-// whose exponents bound the product's (|silu(g)| <= |g|), so they agree on the
-// row's factor; the few bits by which the bound is too large come off a range
-// of 2^-24 below 2^15.
+// workgroup of a row scans all of it for the largest finite product, so they
+// agree on the row's factor.  The scan's products come of the exponential and
+// reciprocal instructions: within 2^-16 of the staged ones, which moves the
+// factor of a row whose maximum lies that close to a power of two, and the
+// largest staged value from [2^14, 2^15) to at most 2^15 (1 + 2^-16).
+// (max|gate| times max|up| in its place loses the row where they lie in
+// different columns or the gate is negative; the products cost 0.3 us of a
+// call of 24 x 1536x8960, 16.3 -> 16.6, and 0.4 of 64 rows, 24.0 -> 24.5.)
 __global__ __launch_bounds__(256) void rows_stage_swiglu_kernel(const void* x, u32x4* out, float* rowscale, int K) {
-    __shared__ uint32_t wmax[2][4];
+    __shared__ float wmax[4];
     const int m = blockIdx.x;
     const int chunks = K / 8;
     const uint16_t* gu = (const uint16_t*)x + (int64_t)m * 2 * K;
     const int own = blockIdx.y * 256 + threadIdx.x;
     float v[8];
     if (own < chunks) stage_load8<kSwiGLU>(x, m, K, own, v);
-    uint32_t mx[2] = {0, 0};  // bf16 magnitude bits
+    float mx = 0.0f;
+    auto largest = [&](uint32_t gate, uint32_t up) {
+        // |g| / (1 + e^-g) |u|; 2^-8 on both sides of the quotient keeps the
+        // reciprocal (of at most 2^128) a normal number
+        const float g = bf16_bits_to_float(gate), u = bf16_bits_to_float(up);
+        const float e = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
+        const float p = (fabsf(g) * 0x1p-8f) * __builtin_amdgcn_rcpf(__builtin_fmaf(e, 0x1p-8f, 0x1p-8f)) * fabsf(u);
+        mx = p < INFINITY ? fmaxf(mx, p) : mx;  // (neither infinite nor NaN)
+    };
     for (int c = threadIdx.x; c < chunks; c += 256) {
+        const u32x4 g = *(const u32x4*)(gu + 8 * c), u = *(const u32x4*)(gu + K + 8 * c);
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const u32x4 d = *(const u32x4*)(gu + (int64_t)p * K + 8 * c);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t lo = d[i] & 0x7FFFu, hi = (d[i] >> 16) & 0x7FFFu;
-                mx[p] = max(mx[p], max(lo < 0x7F80u ? lo : 0u, hi < 0x7F80u ? hi : 0u));
-            }
+        for (int i = 0; i < 4; ++i) {
+            largest(g[i] & 0xFFFFu, u[i] & 0xFFFFu);
+            largest(g[i] >> 16, u[i] >> 16);
         }
     }
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        // (magnitude bits of non-negative bf16 values order as the values do)
-        const float w = wave_max64(bf16_bits_to_float(mx[p]));
-        if ((threadIdx.x & 63) == 0) wmax[p][threadIdx.x >> 6] = __builtin_bit_cast(uint32_t, w);
-    }
+    mx = wave_max64(mx);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
     __syncthreads();
-    int e = 0;
-    bool zero = false;
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const float w = __builtin_bit_cast(float, max(max(wmax[p][0], wmax[p][1]), max(wmax[p][2], wmax[p][3])));
-        int ex;
-        (void)frexpf(w, &ex);  // w = f 2^ex, f in [0.5, 1)
-        e += ex;
-        zero = zero || w == 0.0f;
-    }
-    // products lie below 2^e; a finite one below 2^128
     float inv, rs;
-    row_factors(zero ? 0.0f : ldexpf(0.5f, max(min(e, 128), -125)), inv, rs);
+    row_factors(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])), inv, rs);
     if (threadIdx.x == 0 && blockIdx.y == 0) rowscale[m] = rs;
     if (own < chunks) {
         u32x4 hi, lo;

@@ -573,6 +573,42 @@ def test_few_row_tiles_of_the_swiglu_product(rows, n, k):
     assert bool((y[3] == 0).all()) and not bool(torch.isfinite(y[5]).any())
 
 
+@pytest.mark.parametrize("rows,n,k", [(17, 96, 8960), (40, 200, 128), (100, 264, 1536), (260, 2600, 4160)])
+def test_swiglu_rows_of_unlike_gate_and_up(rows, n, k):
+    """w4g64_linear_swiglu where a row's largest |gate| and |up| say little about
+    its largest product (strongly negative gates; outliers in different columns).
+    Beside the bound of ordinary rows, the two fp16 planes of a row whose largest
+    product is scaled to 2^14 or more end at 2^-25: 2^-39 of it."""
+    from qwen_int4_hip import _lib
+
+    lib = _lib.load()
+    q, s, z = weights("asym", n, k, rows + n)
+    qt, st, zt = dev_weights(q, s, z)
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    gate, up = torch.randn((2, rows, k), generator=gen, device=DEV)
+    own = torch.arange(rows, device=DEV) % 8
+    gate = torch.where((own == 0)[:, None], -30 + gate, gate)         # silu(gate) near 3e-12
+    gate = torch.where((own == 1)[:, None], -20 + gate / 4, gate)
+    gate = torch.where((own == 2)[:, None], -88 + gate.sign() / 2, gate)  # near fp32's smallest normal number ...
+    up = torch.where((own == 2)[:, None], up * 2.0 ** 110, up)        # ... times a large one
+    gate[own == 3, 1], up[own == 3, 2] = -80.0, 2000.0
+    gate[own == 4, k - 1], up[own == 4, 0] = 2.0 ** 20, -2.0 ** 20
+    gate[own == 5, k // 2], up[own == 5, k // 2 + 1] = -(2.0 ** 100), 2.0 ** 60
+    gate[own == 6, 3] = -(2.0 ** 90)
+    gu = torch.cat((gate, up), dim=1).to(torch.bfloat16)
+    y = torch.empty((rows, n), device=DEV)
+    need = lib.w4g64_linear_workspace_bytes(rows, n, k, _lib.DTYPE_BF16_SWIGLU)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    _lib.check(lib.w4g64_linear_swiglu(ptr(gu), ptr(qt), ptr(st), ptr(zt), None, 0, ptr(y), rows, n, k, ptr(ws), need,
+                                       ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    w = dequantize_canonical_w4g64_hip(qt, st, zt, out_features=n, in_features=k).double()
+    h = torch.nn.functional.silu(gu[:, :k].double()) * gu[:, k:].double()
+    bound = (h.abs() @ w.abs().t()) * 2.0 ** -20 + h.abs().amax(1, keepdim=True) * w.abs().sum(1) * 2.0 ** -39
+    err = (y.double() - h @ w.t()).abs() / bound
+    assert bool((err <= 1).all()), {i: err[own == i].max().item() for i in range(8)}
+
+
 @pytest.mark.parametrize(
     ("rows", "n", "k"),
     [(65, 72, 64),        # one group: two steps; the second half holds one row
