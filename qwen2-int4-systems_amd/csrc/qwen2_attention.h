@@ -8,6 +8,11 @@
 
 namespace w4g64 {
 
+// Where a softmax's running maximum starts: finite, so that a row whose keys so
+// far all scored -inf (masked, or their products overflowed) adds exp2(-inf) =
+// 0 to its sums, not exp2(-inf + inf), and below every finite score.
+constexpr float kScoreFloor = -3.402823466e+38f;
+
 // Maximum / sum over the four lanes j, j + 16, j + 32, j + 48.  (The swapped
 // pair is bit cast as a whole: a bit cast of one element of the builtin's
 // integer pair compiles to element 0 with this compiler.)

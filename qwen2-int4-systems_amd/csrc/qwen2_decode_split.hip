@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void decode_split_kernel(DecodeSp
     u32x4 qf[4];  // columns past the group repeat its last head and are not stored
     rope_pieces(qkv + (kvh * group + min(j, group - 1)) * kAttnHeadDim, cs, sn, q, qf);
 
-    float m_run = -INFINITY, l_run = 0.0f;
+    float m_run = kScoreFloor, l_run = 0.0f;
     float4v o[8];
 #pragma unroll
     for (int dd = 0; dd < 8; ++dd) o[dd] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kSplitThreads, 2) void decode_split_kernel(DecodeSp
         for (int e = 1; e < 8; ++e) bm = fmaxf(bm, s[e]);
         const float mn = fmaxf(m_run, quarters_max(bm));
         if (__any(mn != m_run)) {
-            const float alpha = __builtin_amdgcn_exp2f(m_run - mn);  // 2^-inf = 0 on the first block
+            const float alpha = __builtin_amdgcn_exp2f(m_run - mn);
             l_run *= alpha;
 #pragma unroll
             for (int dd = 0; dd < 8; ++dd) o[dd] *= alpha;
@@ -231,8 +231,8 @@ __global__ __launch_bounds__(kSplitThreads, 2) void decode_split_kernel(DecodeSp
         }
     }
     __syncthreads();
-    // thread t: head t / 32, dimensions 4 (t % 32) .. + 3.  Wave 0 holds a
-    // block, so the maximum is finite; a wave without one adds exp2(-inf) = 0.
+    // thread t: head t / 32, dimensions 4 (t % 32) .. + 3.  A wave without a
+    // block, or a finite score, adds its sums of zero.
     const int g = tid / 32;
     const int d4 = 4 * (tid % 32);
     if (g >= group) return;

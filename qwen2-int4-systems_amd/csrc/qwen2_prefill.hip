@@ -183,7 +183,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
         *(u32x4*)(queries + r * kRowBytes + 16 * ((tid % 16) ^ (r % 16))) = x ^ a.query_sign;
     }
     __syncthreads();
-    float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.0f, 0.0f};
+    float m_run[2] = {kScoreFloor, kScoreFloor}, l_run[2] = {0.0f, 0.0f};
     bool seen[2] = {false, false};  // kMasked: the row had an allowed key
     float4v o[8][2];
 #pragma unroll
@@ -265,21 +265,19 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
 #pragma unroll
             for (int e = 1; e < 8; ++e) bm = fmaxf(bm, s[u][e]);
             // the sums are rescaled only once a score passes their reference
-            // by 8 units of the base-2 exponent (from -inf on the first
+            // by 8 units of the base-2 exponent (from the floor on the first
             // block); until then probabilities reach 2^8, which changes no
             // relative rounding
             const float mn = quarters_max(bm) * a.scale2;
             if (__any(mn - m_run[u] > 8.0f)) {
                 const float to = fmaxf(m_run[u], mn);
-                float alpha = __builtin_amdgcn_exp2f(m_run[u] - to);  // 2^-inf = 0 on the first block
-                if (kMasked && to == -INFINITY) alpha = 1.0f;         // (another row's turn: no key here yet)
+                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - to);  // (1 where it is another row's turn)
                 l_run[u] *= alpha;
 #pragma unroll
                 for (int dd = 0; dd < 8; ++dd) o[dd][u] *= alpha;
                 m_run[u] = to;
             }
-            // (a masked row may have met no key yet: 2^-inf, not -inf + inf)
-            const float ref = kMasked && m_run[u] == -INFINITY ? 0.0f : -m_run[u];
+            const float ref = -m_run[u];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float p0 = __builtin_amdgcn_exp2f(fmaf(s[u][2 * e], a.scale2, ref));
@@ -310,7 +308,8 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
     if (blk <= last) step(std::false_type{});
 
     // ---- the waves' results meet in LDS: waves 2 and 3 give theirs to 0 and
-    // 1, then wave 1 to wave 0, which stores the rows; a wave without a block (or an allowed key) adds 2^-inf = 0 ----
+    // 1, then wave 1 to wave 0, which stores the rows; a wave without a block
+    // (or an allowed key) adds its sums of zero ----
     float l_all[2] = {quarters_sum(l_run[0]), quarters_sum(l_run[1])};
     float(*so)[kTile][kOutStride] = (float(*)[kTile][kOutStride])smem;
 #pragma unroll
@@ -341,9 +340,8 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
             for (int u = 0; u < 2; ++u) {
                 const float mo = sm[wave][16 * u + j];
                 const float to = fmaxf(m_run[u], mo);
-                // (waves 1 and 3 may both be without a block)
-                const float f = to == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run[u] - to);
-                const float fo = to == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mo - to);
+                const float f = __builtin_amdgcn_exp2f(m_run[u] - to);
+                const float fo = __builtin_amdgcn_exp2f(mo - to);
                 m_run[u] = to;
                 seen[u] = seen[u] || sn[wave][16 * u + j] != 0;
                 l_all[u] = fmaf(sl[wave][16 * u + j], fo, l_all[u] * f);

@@ -452,6 +452,67 @@ def test_prefill_attention_block_edges(batch, heads, kv_heads, length, max_lengt
     assert bool((err <= bound).all()), (err - bound).max().item()
 
 
+@pytest.mark.parametrize("length,low", [(70, ((0, 32),)), (200, ((0, 32), (96, 128), (160, 165)))])
+def test_prefill_attention_keys_of_infinite_score(length, low):
+    """Keys whose scores overflow to -inf in fp32 take no part, also where they
+    fill a wave's first 32-key block (bound as in the block edges' test)."""
+    lib = _lib.load()
+    g = _gen(length)
+    d, heads, kv_heads = 128, 4, 2
+    q, k, v = (torch.randn((length, h, d), generator=g, device="cuda").to(torch.bfloat16)
+               for h in (heads, kv_heads, kv_heads))
+    q[:, :, 0] = 100.0
+    dead = torch.zeros(length, dtype=torch.bool, device="cuda")
+    for begin, end in low:
+        dead[begin:end] = True
+    k[dead, :, 0] = -3e38
+    qkv = torch.cat((q, k, v), dim=1).reshape(length, -1).contiguous()
+    cos, sin = torch.ones((length, d), dtype=torch.bfloat16, device="cuda"), torch.zeros((length, d), dtype=torch.bfloat16, device="cuda")
+    caches = torch.zeros((2, 1, kv_heads, length, d), dtype=torch.bfloat16, device="cuda")
+    out = torch.empty((length, heads * d), dtype=torch.bfloat16, device="cuda")
+    ws = torch.empty(lib.qwen2_prefill_attention_workspace_bytes(1, heads, length), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.qwen2_prefill_attention(
+        _p(qkv), _p(cos), _p(sin), _p(caches[0]), _p(caches[1]), _p(out), 1, length, heads, kv_heads, d, length,
+        ctypes.c_float(d ** -0.5), _p(ws), ws.numel(), _stream()))
+    kk, vv = (t.double().repeat_interleave(heads // kv_heads, dim=1).transpose(0, 1).contiguous() for t in (k, v))
+    scores = torch.matmul(q.double().transpose(0, 1).contiguous(), kk.transpose(-1, -2).contiguous()) * d ** -0.5
+    causal = torch.ones((length, length), dtype=torch.bool, device="cuda").tril()
+    allowed = causal & ~dead
+    live = allowed.any(-1)  # rows with a finite score
+    probs = torch.softmax(scores.masked_fill(~allowed, float("-inf"))[:, live], dim=-1)
+    want = torch.matmul(probs, vv).transpose(0, 1).reshape(-1, heads * d)
+    err = (out[live].double() - want).abs()
+    bound = want.abs() * 2.0 ** -8 + want.abs().max() * 2.0 ** -16 * (1 + scores[:, live][:, :, ~dead].abs().max())
+    assert bool((err <= bound).all()), (err - bound).max().item()
+
+
+@pytest.mark.parametrize("max_length,pos,dead", [(64, 60, 32), (64, 63, 63), (1100, 1000, 900), (4096, 4095, 4000)])
+def test_decode_attention_keys_of_infinite_score(max_length, pos, dead):
+    """The split kernel where whole waves and splits meet nothing but scores of -inf."""
+    lib = _lib.load()
+    g = _gen(max_length + pos)
+    d, heads, kv_heads, batch = 128, 4, 2, 2
+    k_cache, v_cache = (torch.randn((batch, kv_heads, max_length, d), generator=g, device="cuda").to(torch.bfloat16)
+                        for _ in range(2))
+    k_cache[:, :, :dead, 0] = float("-inf")
+    qkv = torch.randn((batch, heads + 2 * kv_heads, d), generator=g, device="cuda").to(torch.bfloat16)
+    qkv[:, :heads, 0] = 100.0
+    cos, sin = torch.ones((batch, d), dtype=torch.bfloat16, device="cuda"), torch.zeros((batch, d), dtype=torch.bfloat16, device="cuda")
+    out = torch.empty((batch, heads * d), dtype=torch.bfloat16, device="cuda")
+    ws = torch.zeros(lib.qwen2_decode_attention_workspace_bytes(batch, kv_heads, max_length), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.qwen2_decode_attention(
+        _p(qkv), _p(cos), _p(sin), _p(k_cache), _p(v_cache), _p(torch.tensor([pos], device="cuda")), _p(out), batch,
+        heads, kv_heads, d, max_length, ctypes.c_float(d ** -0.5), _p(ws), ws.numel(), _stream()))
+    keys = torch.cat((k_cache[:, :, :pos], qkv[:, heads:heads + kv_heads, None]), dim=2)[:, :, dead:].double()
+    values = torch.cat((v_cache[:, :, :pos], qkv[:, heads + kv_heads:, None]), dim=2)[:, :, dead:].double()
+    q = qkv[:, :heads].reshape(batch, kv_heads, -1, 1, d).double()
+    scores = (q * keys.unsqueeze(2)).sum(-1) * d ** -0.5
+    want = (torch.softmax(scores, dim=-1) @ values).reshape(batch, heads * d)
+    err = (out.double() - want).abs()
+    bound = want.abs() * 2.0 ** -8 + want.abs().max() * 2.0 ** -16 * (1 + scores.abs().max())
+    assert bool((err <= bound).all()), (err - bound).max().item()
+
+
 @pytest.mark.parametrize("batch,heads,kv_heads,length,past,masking", [
     (1, 12, 2, 1, 0, "none"),        # one row, its own key only
     (4, 12, 2, 33, 0, "left"),       # left-padded prompts: rows without an allowed key
