@@ -28,6 +28,7 @@
 //
 // The new key at position p is read by the chunk that holds p from LDS, never
 // from the cache, so no workgroup reads a cache row another one is writing.
+#include <float.h>
 #include <math.h>
 #include <stdarg.h>
 
@@ -731,6 +732,15 @@ int64_t qwen2_prefill_attention_workspace_bytes(int64_t batch, int64_t num_heads
     return batch * num_heads * length * kHeadDim * (int64_t)sizeof(uint16_t);
 }
 
+// The prompt kernel scales scores it has masked with -inf, so its scale must
+// not be zero: the smallest normal number leaves every score below 2^102 a
+// weight of exactly one, as zero would.
+static void set_scale(PrefillArgs& args, float scale) {
+    const float s = fabsf(scale) * 1.4426950408889634f;
+    args.scale2 = s < FLT_MIN ? FLT_MIN : s;
+    args.query_sign = scale < 0.0f ? 0x80008000u : 0u;
+}
+
 int qwen2_prefill_attention(const void* qkv, const void* cos, const void* sin, void* k_cache, void* v_cache,
                             void* out, int64_t batch, int64_t length, int64_t num_heads, int64_t num_kv_heads,
                             int64_t head_dim, int64_t max_length, float scale, void* workspace,
@@ -774,8 +784,7 @@ int qwen2_prefill_attention(const void* qkv, const void* cos, const void* sin, v
     args.heads = (int)num_heads;
     args.kv_heads = (int)num_kv_heads;
     args.max_len = (int)max_length;
-    args.scale2 = fabsf(scale) * 1.4426950408889634f;
-    args.query_sign = scale < 0.0f ? 0x80008000u : 0u;
+    set_scale(args, scale);
     return launch_status(launch_prefill_attention(args, (hipStream_t)stream), "prefill_attention");
 }
 
@@ -820,8 +829,7 @@ int qwen2_cached_attention(const void* q, const void* k, const void* v, const vo
     args.heads = (int)num_heads;
     args.kv_heads = (int)num_kv_heads;
     args.max_len = (int)total;
-    args.scale2 = fabsf(scale) * 1.4426950408889634f;
-    args.query_sign = scale < 0.0f ? 0x80008000u : 0u;
+    set_scale(args, scale);
     return launch_status(launch_prefill_attention(args, (hipStream_t)stream), "cached_attention");
 }
 

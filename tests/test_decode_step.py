@@ -513,6 +513,28 @@ def test_decode_attention_keys_of_infinite_score(max_length, pos, dead):
     assert bool((err <= bound).all()), (err - bound).max().item()
 
 
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-42])
+@pytest.mark.parametrize("length", [5, 70])
+def test_prefill_attention_without_scale(length, scale):
+    """A scale of zero (or too small for a normal number) is the mean of the
+    values so far: exact bf16 weights of one, fp32 sums."""
+    lib = _lib.load()
+    d, heads, kv_heads = 128, 4, 2
+    qkv = torch.randn((length, (heads + 2 * kv_heads) * d), generator=_gen(length), device="cuda").to(torch.bfloat16)
+    cos, sin = RotaryEmbedding(d, 1_000_000.0).cuda()(torch.arange(length, device="cuda"), torch.bfloat16)
+    caches = torch.zeros((2, 1, kv_heads, length, d), dtype=torch.bfloat16, device="cuda")
+    out = torch.empty((length, heads * d), dtype=torch.bfloat16, device="cuda")
+    ws = torch.empty(lib.qwen2_prefill_attention_workspace_bytes(1, heads, length), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.qwen2_prefill_attention(
+        _p(qkv), _p(cos), _p(sin), _p(caches[0]), _p(caches[1]), _p(out), 1, length, heads, kv_heads, d, length,
+        ctypes.c_float(scale), _p(ws), ws.numel(), _stream()))
+    values = qkv[:, (heads + kv_heads) * d:].double().view(length, kv_heads, 1, d).expand(-1, -1, heads // kv_heads, d)
+    count = torch.arange(1, length + 1, device="cuda").double().view(-1, 1, 1, 1)
+    want = (values.cumsum(0) / count).reshape(length, heads * d)
+    err = (out.double() - want).abs()
+    assert bool((err <= want.abs() * 2.0 ** -8 + want.abs().max() * 2.0 ** -16).all()), err.max().item()
+
+
 @pytest.mark.parametrize("batch,heads,kv_heads,length,past,masking", [
     (1, 12, 2, 1, 0, "none"),        # one row, its own key only
     (4, 12, 2, 33, 0, "left"),       # left-padded prompts: rows without an allowed key
