@@ -245,9 +245,9 @@ def cached_attention_hip(q, k, v, cos, sin, past, mask, *, num_heads: int, num_k
     ``q`` [B, S, H * 128], ``k``, ``v`` [B, S, KVH * 128] projections, ``cos``,
     ``sin`` [B, S, 128], ``past`` None or (key, value) [B, KVH, P, 128], ``mask``
     [B, P + S] (zero: excluded).  Returns the attended rows [B, S, H * 128] and
-    the new (key, value) cache.  None, with nothing done, for tensors it does
-    not take: other types or devices, another head dimension, a gradient to be
-    recorded, subclasses and modes.
+    the new (key, value) cache.  None, with nothing done, for what it does not
+    take: tensors of other types, shapes or devices, a gradient to be recorded,
+    subclasses and modes.
     """
     tensors = (q, k, v, cos, sin) + (() if past is None else tuple(past))
     device = q.device
@@ -263,9 +263,10 @@ def cached_attention_hip(q, k, v, cos, sin, past, mask, *, num_heads: int, num_k
             or mask.device != device or not batch * length
             or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))):
         return None
-    length_past = 0 if past is None else past[0].shape[2]
+    length_past = 0 if past is None or past[0].ndim != 4 else past[0].shape[2]
     total = length_past + length
-    if tuple(mask.shape) != (batch, total):
+    if (tuple(mask.shape) != (batch, total)
+            or past is not None and [tuple(t.shape) for t in past] != 2 * [(batch, num_kv_heads, length_past, 128)]):
         return None
     # (contiguous and aligned already where the linears and this function made them)
     q, k, v, cos, sin = (t.contiguous() for t in (q, k, v, cos, sin))

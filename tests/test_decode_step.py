@@ -591,6 +591,28 @@ def test_cached_attention_matches_torch(batch, heads, kv_heads, length, past, ma
     assert bool((out[blind] == 0).all())
 
 
+def test_cached_attention_takes_no_past_of_another_shape():
+    """A past that the kernels would read out of its bounds is left to torch."""
+    from qwen_int4_hip.kernels import cached_attention_hip
+
+    q, kv = (torch.randn((2, 3, h * 128), device="cuda").to(torch.bfloat16) for h in (4, 2))
+    cos = torch.ones((2, 3, 128), device="cuda", dtype=torch.bfloat16)
+    mask = torch.ones((2, 10), device="cuda", dtype=torch.bool)
+
+    def past(*shape):
+        return torch.zeros(shape, device="cuda", dtype=torch.bfloat16)
+
+    def call(*caches):
+        return cached_attention_hip(q, kv, kv, cos, cos, caches, mask, num_heads=4, num_kv_heads=2)
+
+    whole = past(2, 2, 7, 128)
+    for caches in ((past(2, 1, 7, 128), whole), (whole, past(2, 1, 7, 128)), (past(2, 2, 7, 64),) * 2,
+                   (whole, past(2, 2, 6, 128)), (past(1, 2, 7, 128),) * 2, (past(2, 2, 7),) * 2, (whole,) * 3,
+                   (past(2, 4, 7, 128),) * 2):
+        assert call(*caches) is None, [tuple(t.shape) for t in caches]
+    assert call(whole, whole) is not None
+
+
 def test_cached_attention_leaves_other_tensors_to_torch():
     from qwen_int4_hip.kernels import cached_attention_hip
 
