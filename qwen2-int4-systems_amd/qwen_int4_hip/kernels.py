@@ -239,6 +239,16 @@ def linear_kernel_name(rows: int, out_features: int, in_features: int, dtype: to
     return _lib.load().w4g64_linear_kernel_name(rows, out_features, in_features, _DTYPE_CODE[dtype]).decode()
 
 
+def _operators_followed() -> bool:
+    """Whether a function or dispatch mode, ``torch.jit.trace``, a functorch
+    level, forward-mode differentiation or ``torch.compile`` follows torch's
+    operators, which see nothing of a call into the library."""
+    return (torch.compiler.is_compiling() or torch._C._len_torch_function_stack() > 0
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
 def cached_attention_hip(q, k, v, cos, sin, past, mask, *, num_heads: int, num_kv_heads: int):
     """Rotary step, cache concatenation, masking and attention of
     ``QwenAttention.forward`` (src/qwen_int4/model.py:61-122) on the HIP kernels:
@@ -246,9 +256,11 @@ def cached_attention_hip(q, k, v, cos, sin, past, mask, *, num_heads: int, num_k
     ``sin`` [B, S, 128], ``past`` None or (key, value) [B, KVH, P, 128], ``mask``
     [B, P + S] (zero: excluded).  Returns the attended rows [B, S, H * 128] and
     the new (key, value) cache.  None, with nothing done, for what it does not
-    take: tensors of other types, shapes or devices, a gradient to be recorded,
-    subclasses and modes.
+    take: tensors of other types, shapes or devices, subclasses, a gradient to
+    be recorded, and where something follows torch's operators.
     """
+    if _operators_followed():
+        return None
     tensors = (q, k, v, cos, sin) + (() if past is None else tuple(past))
     device = q.device
     if q.ndim != 3 or any(type(t) is not torch.Tensor or t.dtype is not torch.bfloat16 or t.device != device

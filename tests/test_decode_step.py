@@ -592,7 +592,12 @@ def test_cached_attention_matches_torch(batch, heads, kv_heads, length, past, ma
 
 
 def test_cached_attention_takes_no_past_of_another_shape():
-    """A past that the kernels would read out of its bounds is left to torch."""
+    """A past that the kernels would read out of its bounds, and states in which
+    torch's operators are followed, are left to torch."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
     from qwen_int4_hip.kernels import cached_attention_hip
 
     q, kv = (torch.randn((2, 3, h * 128), device="cuda").to(torch.bfloat16) for h in (4, 2))
@@ -610,6 +615,9 @@ def test_cached_attention_takes_no_past_of_another_shape():
                    (whole, past(2, 2, 6, 128)), (past(1, 2, 7, 128),) * 2, (past(2, 2, 7),) * 2, (whole,) * 3,
                    (past(2, 4, 7, 128),) * 2):
         assert call(*caches) is None, [tuple(t.shape) for t in caches]
+    for mode in (TorchFunctionMode(), TorchDispatchMode(), forward_ad.dual_level()):
+        with mode:
+            assert call(whole, whole) is None, type(mode)
     assert call(whole, whole) is not None
 
 

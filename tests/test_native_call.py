@@ -119,3 +119,21 @@ def test_native_call_leaves_other_forms_to_the_general_route(marks):
     torch.func.vmap(lambda t: (seen.append(_native(x, weights)), seen.append(_native(t, weights)), t)[2])(x)
     torch.jit.trace(lambda t: (seen.append(_native(t, weights)), t + 0)[1], (x,), check_trace=False)
     assert len(seen) >= 3 and all(y is None for y in seen)
+
+
+def test_what_follows_torch_operators_is_seen():
+    """The states in which the attention layer keeps to torch's operators."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    assert not kernels._operators_followed()
+    for mode in (TorchFunctionMode(), TorchDispatchMode(), forward_ad.dual_level()):
+        with mode:
+            assert kernels._operators_followed(), type(mode)
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(kernels._operators_followed()), t)[1])(torch.zeros(2))
+    torch.jit.trace(lambda t: (seen.append(kernels._operators_followed()), t + 0)[1], (torch.zeros(2),), check_trace=False)
+    compiled = torch.compile(lambda t: t + int(kernels._operators_followed()), backend="eager")(torch.zeros(2))
+    assert len(seen) >= 2 and all(seen) and compiled.tolist() == [1, 1]
+    assert not kernels._operators_followed()
