@@ -118,7 +118,8 @@ class QwenAttention(nn.Module):
         (``QwenModel`` always passes one).  What the tensors themselves rule
         out, ``cached_attention_hip`` answers."""
         return (self.head_dim == 128 and attention_mask is not None and torch.cuda.is_available()
-                and all(p.backend == "hip" for p in (self.q_proj, self.k_proj, self.v_proj, self.o_proj)))
+                and all(getattr(p, "backend", None) == "hip"
+                        for p in (self.q_proj, self.k_proj, self.v_proj, self.o_proj)))
 
     def _output(self, attended, batch, sequence):
         return self.o_proj(attended.transpose(1, 2).contiguous().view(batch, sequence, self.num_heads * self.head_dim))

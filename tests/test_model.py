@@ -286,3 +286,20 @@ def test_full_workload_fused_serving_path_against_reference_backend():
     print(f"greedy choices: {int(clear.sum())} of {steps + 1} clear of the logit error; {agree:.1%} agree overall")
     assert int(clear.sum()) >= 8
     assert torch.equal(picked[clear], ref_tokens[clear])
+
+
+def test_attention_layer_takes_projections_of_another_kind(monkeypatch):
+    """A projection replaced by any other module (here ``nn.Linear``) runs."""
+    from qwen_int4_hip import PackingFormat
+    from qwen_int4_hip.model import QwenAttention
+
+    config = SimpleNamespace(hidden_size=256, num_attention_heads=2, num_key_value_heads=1)
+    layer = QwenAttention(config, backend="torch", packing=PackingFormat.CANONICAL, group_size=64)
+    for name in ("q_proj", "k_proj", "v_proj", "o_proj"):
+        proj = getattr(layer, name)
+        setattr(layer, name, torch.nn.Linear(proj.in_features, proj.out_features, dtype=torch.bfloat16))
+    hidden, factors = torch.randn(1, 3, 256).bfloat16(), torch.ones(1, 3, 128).bfloat16()
+    with torch.no_grad():
+        want = layer(hidden, factors, factors, torch.ones(1, 3))[0]
+        monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+        assert torch.equal(layer(hidden, factors, factors, torch.ones(1, 3))[0], want)
