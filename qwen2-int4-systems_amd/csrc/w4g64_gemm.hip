@@ -947,9 +947,11 @@ const char* gemm_kernel_name(int64_t rows, int64_t out_features, int64_t in_feat
 hipError_t launch_gemm(const LinearProblem& p, void* workspace, int64_t workspace_bytes, hipStream_t stream,
                        hipEvent_t start, hipEvent_t stop) {
     const RowsPlan few = plan_rows(p.rows, p.out_features, p.in_features, p.x_kind);
-    if (few.taken && few.workspace_bytes <= workspace_bytes) return launch_rows(p, few, workspace, stream, start, stop);
     const GemmLayout l = gemm_layout(p.rows, p.out_features, p.in_features, p.x_kind);
     const GemmPlan& pl = l.plan;
+    // (the problem chooses: a larger buffer than the query's changes nothing)
+    if (few_rows_fit(few, l.bytes) && few.workspace_bytes <= workspace_bytes)
+        return launch_rows(p, few, workspace, stream, start, stop);
     const bool two = two_planes(p.x_kind);
     uint16_t* staged = (uint16_t*)((char*)workspace + l.staged_offset);
     float* rowscale = (float*)((char*)workspace + l.rowscale_offset);

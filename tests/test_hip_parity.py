@@ -638,6 +638,31 @@ def test_row_blocks(rows, n, k, dtype):
     test_few_row_tiles(rows, n, k, dtype)
 
 
+@pytest.mark.parametrize("rows,n,k,dtype", [
+    (1554, 1330, 1344, "bf16"),  # row blocks of more than the static scratch, tiles of less: the tiles
+    (300, 520, 1536, "bf16"),    # row blocks
+    (160, 1536, 1536, "fp32"),
+])
+def test_gemm_is_chosen_by_the_problem_alone(rows, n, k, dtype):
+    """The same bits from a workspace of the queried size and from a larger one."""
+    from qwen_int4_hip import _lib
+
+    lib = _lib.load()
+    qt, st, zt = dev_weights(*weights("sym", n, k, rows))
+    x = to_dev(O.activations(rows, k, seed=rows, dtype=dtype), dtype)
+    code = {"bf16": _lib.DTYPE_BF16, "fp32": _lib.DTYPE_F32}[dtype]
+    need = lib.w4g64_linear_workspace_bytes(rows, n, k, code)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    got = []
+    for size in (need, need + (32 << 20)):
+        ws = torch.empty(size, dtype=torch.uint8, device=DEV)
+        y = torch.empty((rows, n), dtype=x.dtype, device=DEV)
+        _lib.check(lib.w4g64_linear(ptr(x), code, ptr(qt), ptr(st), ptr(zt), None, 0, ptr(y), rows, n, k, ptr(ws),
+                                    size, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got.append(y)
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("rows,n,k", [(70, 72, 64), (160, 520, 1984), (260, 2600, 4160)])
 def test_two_planes_of_the_swiglu_product(rows, n, k):
     test_few_row_tiles_of_the_swiglu_product(rows, n, k)
