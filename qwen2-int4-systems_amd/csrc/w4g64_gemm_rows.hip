@@ -67,6 +67,14 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Order of a wave's own LDS accesses, lane to lane: the hardware keeps it, this
+// tells the compiler.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 template <int XK, int THREADS>
 __global__ __launch_bounds__(THREADS) void rows_stage_kernel(const void* x, u32x4* out, float* rowscale, int K) {
     constexpr int kPlanes = XK == kF32 ? 2 : 1;
@@ -288,9 +296,11 @@ __global__ __launch_bounds__(64 * W) void rows_gemm_kernel(RowsArgs a) {
                 for (int r = 0; r < 4; ++r) acc[m][c][r] = __builtin_fmaf(sc[c], d[r], acc[m][c][r]);
             }
     };
-    auto put_w = [&](const u32x4 (&w)[CT]) {
+    auto put_w = [&](const u32x4 (&w)[CT]) {  // after the last pair's reads, before this one's
+        wave_lds_order();
 #pragma unroll
         for (int c = 0; c < CT; ++c) *(u32x4*)(w_put + 1024 * c) = w[c];
+        wave_lds_order();
     };
     Rows x0, x1;
     u32x4 w[CT];
