@@ -34,7 +34,11 @@
 // ballot; blocks without an excluded key or a causal edge take no masking
 // instructions.  With the rotary step and the cache's concatenation in the
 // first launch it replaced some 30 torch launches: a layer over four prompts
-// of up to 300 tokens 401 -> 119 us, of which its four linears take 90.
+// of up to 300 tokens 401 -> 119 us, of which its four linears took 90 then.
+// It replaced fp32 probabilities, so it splits them into three bf16 terms, all
+// of their bits (the prompt's form keeps the two of the kernel before it):
+// 1.2e-4 of the outputs are then not the exact value's rounding, 1.5e-3 with
+// two terms, 1.7e-4 with torch in fp32; the layer 93.0 -> 93.6 us.
 #include <math.h>
 
 #include <type_traits>
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
                     if (16 * (e / 4) + 4 * q + e % 4 > 16 * u + j) s[u][e] = -INFINITY;
         }
         // online softmax (base 2) of the lane's two query rows
-        u32x4 ph[2], pl[2];
+        u32x4 ph[2], pl[2], pt[2];  // probabilities: bf16 hi + lo, kMasked a third term (all 24 bits)
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             float bm = s[u][0];
@@ -284,7 +288,9 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
                 const float p1 = __builtin_amdgcn_exp2f(fmaf(s[u][2 * e + 1], a.scale2, ref));
                 l_run[u] += p0 + p1;
                 ph[u][e] = pack_bf16x2(p0, p1);
-                pl[u][e] = pack_bf16x2(p0 - bf16_lo(ph[u][e]), p1 - bf16_hi(ph[u][e]));
+                const float r0 = p0 - bf16_lo(ph[u][e]), r1 = p1 - bf16_hi(ph[u][e]);
+                pl[u][e] = pack_bf16x2(r0, r1);
+                if constexpr (kMasked) pt[u][e] = pack_bf16x2(r0 - bf16_lo(pl[u][e]), r1 - bf16_hi(pl[u][e]));
             }
         }
 #pragma unroll
@@ -301,6 +307,12 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
             for (int u = 0; u < 2; ++u)
                 o[dd][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vt),
                                                                    __builtin_bit_cast(bf16x8, pl[u]), o[dd][u], 0, 0, 0);
+            if constexpr (kMasked) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    o[dd][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, vt), __builtin_bit_cast(bf16x8, pt[u]), o[dd][u], 0, 0, 0);
+            }
         }
         if constexpr (kMore) load_v(blk + kWaves);
     };

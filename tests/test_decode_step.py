@@ -591,6 +591,35 @@ def test_cached_attention_matches_torch(batch, heads, kv_heads, length, past, ma
     assert bool((out[blind] == 0).all())
 
 
+@pytest.mark.parametrize("batch,length,past", [(4, 300, 0), (6, 1, 1500)])
+def test_cached_attention_keeps_the_probabilities_bits(batch, length, past):
+    """Probabilities of fp32: sums of some hundred products then err by about
+    2^-21 of the value, and an output is another bf16 value (spacing 2^-8 or
+    more) than the exact result's for one in 2^12 of them.  Of 16 bits (2^-17)
+    it would be one in 2^9."""
+    from qwen_int4_hip.kernels import cached_attention_hip
+
+    g = _gen(length + past)
+    d, heads, kv_heads, total = 128, 12, 2, length + past
+    q, k, v = (torch.randn((batch, length, h * d), generator=g, device="cuda").to(torch.bfloat16)
+               for h in (heads, kv_heads, kv_heads))
+    cache = None
+    if past:
+        cache = tuple(torch.randn((2, batch, kv_heads, past, d), generator=g, device="cuda").to(torch.bfloat16))
+    mask = torch.ones((batch, total), dtype=torch.bool, device="cuda")
+    positions = torch.arange(past, total, device="cuda").expand(batch, length)
+    cos, sin = RotaryEmbedding(d, 1_000_000.0).cuda()(positions, torch.bfloat16)
+    out, (keys, values) = cached_attention_hip(q, k, v, cos, sin, cache, mask, num_heads=heads, num_kv_heads=kv_heads)
+    qr = q.view(batch, length, heads, d).transpose(1, 2)
+    qr = qr * cos.unsqueeze(1) + rotate_half(qr) * sin.unsqueeze(1)
+    keys, values = (t.double().repeat_interleave(heads // kv_heads, dim=1) for t in (keys, values))
+    allowed = torch.ones((length, total), dtype=torch.bool, device="cuda").tril(past)
+    scores = torch.matmul(qr.double(), keys.transpose(-1, -2).contiguous()) * d ** -0.5
+    probs = torch.softmax(scores.masked_fill(~allowed, float("-inf")), dim=-1)
+    want = torch.matmul(probs, values).transpose(1, 2).reshape(batch, length, heads * d).to(torch.bfloat16)
+    assert (out != want).float().mean().item() <= 2.0 ** -11
+
+
 def test_cached_attention_takes_no_past_of_another_shape():
     """A past that the kernels would read out of its bounds, and states in which
     torch's operators are followed, are left to torch."""
