@@ -74,7 +74,8 @@ def build_host() -> Path:
 
     root = Path(torch.__file__).resolve().parent
     tmp = HOST_MODULE.with_suffix(".so.tmp")
-    cmd = [shutil.which("g++") or "g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-w",
+    compiler = shutil.which("g++") or str(Path(hipcc()).resolve().parent / "amdclang++")
+    cmd = [compiler, "-std=c++17", "-O2", "-fPIC", "-shared", "-w",
            "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{sysconfig.get_paths()['include']}", f"-I{root / 'include'}",
            f"-I{root / 'include/torch/csrc/api/include'}", f"-I{Path(hipcc()).resolve().parents[1] / 'include'}",

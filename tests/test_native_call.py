@@ -137,3 +137,29 @@ def test_what_follows_torch_operators_is_seen():
     compiled = torch.compile(lambda t: t + int(kernels._operators_followed()), backend="eager")(torch.zeros(2))
     assert len(seen) >= 2 and all(seen) and compiled.tolist() == [1, 1]
     assert not kernels._operators_followed()
+
+
+@pytest.fixture
+def no_host_module(monkeypatch):
+    import sys
+
+    import qwen_int4_hip
+
+    monkeypatch.setattr(_lib, "_host_linear", None)
+    monkeypatch.delattr(qwen_int4_hip, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "qwen_int4_hip._host", None)  # its import fails
+
+
+def test_host_module_that_does_not_load_leaves_all_calls(no_host_module):
+    with pytest.warns(RuntimeWarning, match="general route"):
+        assert _native(torch.zeros(2, K, dtype=torch.float16), _weights("cpu")) is None
+
+
+@pytest.mark.parametrize("marks", [pytest.param(None, marks=gpu)])
+def test_linears_run_without_the_host_module(marks, no_host_module):
+    weights = _weights("cuda")
+    x = torch.randn(4, K, device="cuda", dtype=torch.float16)
+    with pytest.warns(RuntimeWarning, match="general route"):
+        got = hip_w4g64_linear(x, *weights, None, out_features=N, in_features=K, group_size=64,
+                               packing=PackingFormat.CANONICAL)
+    assert torch.equal(got, linear_canonical_w4g64_hip(x, *weights, None))
