@@ -785,6 +785,12 @@ int qwen2_prefill_attention(const void* qkv, const void* cos, const void* sin, v
     args.kv_heads = (int)num_kv_heads;
     args.max_len = (int)max_length;
     set_scale(args, scale);
+    // The attention reads the queries while it writes out, so an out within
+    // qkv's memory (done with once it is rotated, for a caller) needs them elsewhere.
+    const uintptr_t q_begin = (uintptr_t)qkv, o_begin = (uintptr_t)out, rows = (uintptr_t)(batch * length);
+    if (o_begin < q_begin + rows * (uintptr_t)args.q_row * 2 &&
+        q_begin < o_begin + rows * (uintptr_t)(num_heads * kHeadDim) * 2)
+        args.q_copy = (uint16_t*)workspace;
     return launch_status(launch_prefill_attention(args, (hipStream_t)stream), "prefill_attention");
 }
 

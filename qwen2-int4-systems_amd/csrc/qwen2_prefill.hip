@@ -98,6 +98,15 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(PrefillArgs a, int64
         *(u32x4*)(cache + to) = *(const u32x4*)(vec + d);
 }
 
+// The queries of rows q_row apart into rows of their own, 16 bytes per thread.
+__global__ __launch_bounds__(256) void prefill_queries_kernel(PrefillArgs a, int64_t pieces) {
+    const int64_t at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (at >= pieces) return;
+    const int per = a.heads * (kAttnHeadDim / 8);
+    const int64_t row = at / per;
+    *(u32x4*)(a.q_copy + 8 * at) = *(const u32x4*)(a.q + row * a.q_row + 8 * (at - row * per));
+}
+
 // kMasked: the queries follow `past` cached positions, and a key may be excluded
 // for a whole sequence (mask); a row without an allowed key gives zeros.
 template <bool kMasked>
@@ -389,7 +398,16 @@ __global__ __launch_bounds__(kThreads, 3) void prefill_attention_kernel(PrefillA
 
 }  // namespace
 
-hipError_t launch_prefill_attention(const PrefillArgs& args, hipStream_t stream) {
+hipError_t launch_prefill_attention(PrefillArgs args, hipStream_t stream) {
+    if (args.q_copy) {
+        const int64_t copied = (int64_t)args.batch * args.length * args.heads * (kAttnHeadDim / 8);
+        hipLaunchKernelGGL(prefill_queries_kernel, dim3((unsigned)((copied + 255) / 256)), dim3(256), 0, stream, args,
+                           copied);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) return err;
+        args.q = args.q_copy;
+        args.q_row = (int64_t)args.heads * kAttnHeadDim;
+    }
     const bool masked = args.mask || args.past > 0;
     const int64_t pieces = (int64_t)args.batch * (args.past + args.length) * 2 * args.kv_heads * (kAttnHeadDim / 8);
     const dim3 cgrid((unsigned)((pieces + 255) / 256));

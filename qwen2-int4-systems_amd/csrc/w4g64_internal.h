@@ -182,8 +182,9 @@ struct PrefillArgs {
     int max_len;
     float scale2;         // |scale| * log2(e): the softmax runs in base 2
     uint32_t query_sign;  // sign bits of two bf16 queries, set for a negative scale
+    uint16_t* q_copy;     // not null: out overlaps q, which is copied here first
 };
-hipError_t launch_prefill_attention(const PrefillArgs& args, hipStream_t stream);
+hipError_t launch_prefill_attention(PrefillArgs args, hipStream_t stream);
 
 // Chunks the attention-merge form of the pipelined GEMV takes (the cache's
 // max_length up to 1024 positions): it loads every chunk's partial result.
