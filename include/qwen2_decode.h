@@ -105,7 +105,8 @@ int qwen2_decode_attention_partials(const void* qkv, const void* cos, const void
                                     void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Bytes of workspace qwen2_prefill_attention must be given: bf16 [batch,
- * num_heads, length, head_dim] (checked; written only where out overlaps qkv). */
+ * num_heads, length, head_dim] (checked; written only where out overlaps qkv,
+ * any allocation of that size serves elsewhere, qkv itself among them). */
 int64_t qwen2_prefill_attention_workspace_bytes(int64_t batch, int64_t num_heads, int64_t length);
 
 /* Attention over a prompt of `length` positions per sequence.
@@ -121,7 +122,7 @@ int64_t qwen2_prefill_attention_workspace_bytes(int64_t batch, int64_t num_heads
  * with fp32 scores, softmax and sums (causal mask).  head_dim == 128,
  * num_heads / num_kv_heads <= 8, length <= max_length; qkv, the caches and
  * the workspace 16-byte aligned.  out may overlap qkv (the queries then go
- * through the workspace, which must overlap neither).
+ * through the workspace, which then must overlap neither).
  * Replaces: the rotary step, cache update and attention of
  *           QwenAttention.forward over a prompt (src/qwen_int4/model.py:17-31,
  *           :61-122, the causal mask of :94-120). */

@@ -363,10 +363,10 @@ class FusedDecodeStep:
 class FusedPrefill:
     """Prompt pass of ``batch`` unpadded prompts of one length on the HIP
     kernels, filling static caches [batch, kv_heads, max_length, head_dim]:
-    per layer add_rmsnorm, the fused q|k|v GEMM (bias), rotary and causal fp32
-    attention (torch, as ``QwenAttention.forward``), the o_proj GEMM,
+    per layer add_rmsnorm, the fused q|k|v GEMM (bias), rotary, cache update
+    and causal attention (``qwen2_prefill_attention``), the o_proj GEMM,
     add_rmsnorm, the fused gate|up GEMM and the SwiGLU down projection (its
-    product written as the GEMM's bf16 planes; fp32 out).  Returns the
+    product staged as the GEMM's two fp16 planes; fp32 out).  Returns the
     logits [batch, length, vocab] of every prompt position, as the model's
     forward does (src/qwen_int4/model.py:169-199, :231-245)."""
 
@@ -416,8 +416,6 @@ class FusedPrefill:
         cos, sin = cos.reshape(rows, -1).contiguous(), sin.reshape(rows, -1).contiguous()
         h, kvh, d = self.heads, self.kv_heads, self.head_dim
         attended = torch.empty((rows, h * d), dtype=bf16, device=device)
-        qrot = torch.empty(lib.qwen2_prefill_attention_workspace_bytes(batch, h, length) // 2, dtype=bf16,
-                           device=device)
 
         def linear(inp, code, w, out):
             bias = w["bias"]
@@ -435,10 +433,11 @@ class FusedPrefill:
             for layer, fused, (k_cache, v_cache) in zip(model.model.layers, self.fused, caches):
                 norm(delta, delta_code, layer.input_layernorm.weight)
                 linear(normed, _lib.DTYPE_BF16, fused["qkv"], qkv)
-                # rotary, cache update and causal attention in one call
+                # rotary, cache update and causal attention in one call (its
+                # workspace is checked but not touched: the projections are large enough)
                 _lib.check(lib.qwen2_prefill_attention(
                     _ptr(qkv), _ptr(cos), _ptr(sin), _ptr(k_cache), _ptr(v_cache), _ptr(attended), batch, length,
-                    h, kvh, d, k_cache.shape[2], ctypes.c_float(d ** -0.5), _ptr(qrot), qrot.numel() * 2, stream))
+                    h, kvh, d, k_cache.shape[2], ctypes.c_float(d ** -0.5), _ptr(qkv), qkv.numel() * 2, stream))
                 op = layer.self_attn.o_proj
                 linear(attended, _lib.DTYPE_BF16, {"qweight": op.qweight, "scales": op.scales, "zeros": op.zeros,
                                                    "bias": None}, o)

@@ -515,7 +515,8 @@ def test_decode_attention_keys_of_infinite_score(max_length, pos, dead):
 
 @pytest.mark.parametrize("batch,heads,kv_heads,length", [(1, 12, 2, 100), (3, 4, 4, 33)])
 def test_prefill_attention_into_the_projections(batch, heads, kv_heads, length):
-    """The output over qkv's own memory: the same bits as elsewhere."""
+    """The output over qkv's own memory, and qkv as the workspace of an output
+    elsewhere: the same bits."""
     lib = _lib.load()
     d, rows = 128, batch * length
     qkv = torch.randn((rows, (heads + 2 * kv_heads) * d), generator=_gen(length), device="cuda").to(torch.bfloat16)
@@ -524,13 +525,14 @@ def test_prefill_attention_into_the_projections(batch, heads, kv_heads, length):
     ws = torch.empty(lib.qwen2_prefill_attention_workspace_bytes(batch, heads, length), dtype=torch.uint8, device="cuda")
     size = rows * heads * d
     outs = []
-    for at in (None, 0, qkv.numel() - size, qkv.numel() - 64):
+    for at in (None, "workspace", 0, qkv.numel() - size, qkv.numel() - 64):
         memory = torch.cat((qkv.flatten(), torch.zeros(size, dtype=torch.bfloat16, device="cuda")))
-        out = torch.empty(size, dtype=torch.bfloat16, device="cuda") if at is None else memory[at: at + size]
+        elsewhere = at in (None, "workspace")
+        out = torch.empty(size, dtype=torch.bfloat16, device="cuda") if elsewhere else memory[at: at + size]
         caches = torch.zeros((2, batch, kv_heads, length, d), dtype=torch.bfloat16, device="cuda")
         _lib.check(lib.qwen2_prefill_attention(
             _p(memory), _p(cos), _p(sin), _p(caches[0]), _p(caches[1]), _p(out), batch, length, heads, kv_heads, d,
-            length, ctypes.c_float(d ** -0.5), _p(ws), ws.numel(), _stream()))
+            length, ctypes.c_float(d ** -0.5), _p(memory if at == "workspace" else ws), ws.numel(), _stream()))
         outs.append(torch.cat((out, caches.flatten())))
     assert all(torch.equal(o, outs[0]) for o in outs)
 
