@@ -472,7 +472,7 @@ def test_linear_boundary_zero_points_exact(rows):
         np.testing.assert_array_equal(from_dev(got), np.tile(np.array([[-360.0, -1440.0]], np.float32), (rows, 1)))
 
 
-@pytest.mark.parametrize("rows", [1, 7, 16, 48, 200])
+@pytest.mark.parametrize("rows", [1, 7, 16, 48, 200, 2049])  # (2049: the tiled GEMM)
 @pytest.mark.parametrize("dtype", ["fp16", "bf16"])
 def test_one_hot_activations_reproduce_dequantized_weights_exactly(rows, dtype):
     """x = e_k gives y[m, n] = round(W[n, k_m]) -- pins the MFMA operand and
@@ -505,27 +505,16 @@ def test_ragged_shapes(rows, n, k, dtype):
     check_linear(x, q, s, z, bias, n, k, dtype, bias_dtype="fp16")
 
 
-@pytest.mark.parametrize(
-    ("rows", "n", "k"),
-    [(17, 2048, 1536),    # two row tiles, the second nearly empty; eight waves
-     (33, 31, 64),        # one group: one wave has work; a ragged column tile
-     (49, 4112, 704),     # 257 column tiles (four waves), an odd group count
-     (64, 10250, 320),    # two column tiles per workgroup, the last one partial
-     (65, 130, 192),      # tiles 5 -> 6; fp32 past its limit
-     (100, 777, 8960),    # K ranges of 48 groups, the last one shorter; tiles 7 -> 8
-     (128, 96, 10304),    # 161 groups: ranges of at most 160
-     (129, 72, 512)],     # past the limit: the tiled kernel
-)
-@pytest.mark.parametrize("dtype", ["fp16", "bf16", "fp32"])
-def test_few_row_tiles(rows, n, k, dtype):
-    """The GEMM of a few row tiles at the edges of its row tiles, column tiles,
-    K ranges and waves, over a workspace left full of NaN, against the fp64
-    product of the exact weights: fp32 sums of K products of at most 15 |x|
-    carry about sqrt(K) 2^-24 of their size (and the two planes 2^-22 of x),
-    so the result is within its own rounding of the exact one plus 2^-20 of
+def check_exact_products(rows, n, k, dtype, kernel):
+    """A GEMM that runs ``kernel``, over a workspace left full of NaN, against
+    the fp64 product of the exact weights: fp32 sums of K products of at most
+    15 |x| carry about sqrt(K) 2^-24 of their size (and the two planes 2^-22 of
+    x), so the result is within its own rounding of the exact one plus 2^-20 of
     the sum of magnitudes."""
     from qwen_int4_hip import kernels
 
+    torch_dtype = {"fp16": torch.float16, "bf16": torch.bfloat16, "fp32": torch.float32}[dtype]
+    assert kernel in kernels.linear_kernel_name(rows, n, k, torch_dtype)
     q, s, z = weights("asym", n, k, rows + n + k)
     x = O.activations(rows, k, seed=rows + n, dtype=dtype, outliers=True)
     bias = O._from_f32(np.linspace(-0.5, 0.5, n, dtype=np.float32), "bf16")
@@ -542,14 +531,32 @@ def test_few_row_tiles(rows, n, k, dtype):
         (err / size).max().item()
 
 
-@pytest.mark.parametrize("rows,n,k", [(17, 1536, 8960), (40, 200, 128), (64, 96, 2048)])
-def test_few_row_tiles_of_the_swiglu_product(rows, n, k):
-    """w4g64_linear_swiglu at 17..64 rows: the product staged by slices of a row
-    under a common factor (rows of very different size, a row of zeros, one
-    with an infinite gate), against fp64."""
+@pytest.mark.parametrize(
+    ("rows", "n", "k"),
+    [(17, 2048, 1536),    # two row tiles, the second nearly empty; eight waves
+     (33, 31, 64),        # one group: one wave has work; a ragged column tile
+     (49, 4112, 704),     # 257 column tiles (four waves), an odd group count
+     (64, 10250, 320),    # two column tiles per workgroup, the last one partial
+     (65, 130, 192),      # tiles 5 -> 6 in blocks
+     (100, 777, 8960),    # K ranges of 48 groups, the last one shorter; tiles 7 -> 8
+     (128, 96, 10304),    # 161 groups: ranges of at most 160
+     (129, 72, 512)],     # nine tiles
+)
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "fp32"])
+def test_few_row_tiles(rows, n, k, dtype):
+    """The GEMM of a few row tiles at the edges of its row tiles, column tiles,
+    K ranges and waves."""
+    check_exact_products(rows, n, k, dtype, "few rows")
+
+
+def check_swiglu_products(rows, n, k, kernel):
+    """w4g64_linear_swiglu on ``kernel``: the product staged under a common
+    factor of its row (rows of very different size, a row of zeros, one with an
+    infinite gate), against fp64."""
     from qwen_int4_hip import _lib
 
     lib = _lib.load()
+    assert kernel in lib.w4g64_linear_kernel_name(rows, n, k, _lib.DTYPE_BF16_SWIGLU).decode()
     q, s, z = weights("asym", n, k, rows + n)
     qt, st, zt = dev_weights(q, s, z)
     gen = torch.Generator(device=DEV).manual_seed(rows)
@@ -571,6 +578,12 @@ def test_few_row_tiles_of_the_swiglu_product(rows, n, k):
     err = (y.double() - h @ w.t()).abs()
     assert bool((err[keep] <= size[keep] * 2.0 ** -20).all()), (err[keep] / size[keep]).max().item()
     assert bool((y[3] == 0).all()) and not bool(torch.isfinite(y[5]).any())
+
+
+@pytest.mark.parametrize("rows,n,k", [(17, 1536, 8960), (40, 200, 128), (64, 96, 2048), (70, 72, 64),
+                                        (160, 520, 1984)])
+def test_few_row_tiles_of_the_swiglu_product(rows, n, k):
+    check_swiglu_products(rows, n, k, "few rows")
 
 
 @pytest.mark.parametrize("rows,n,k", [(17, 96, 8960), (40, 200, 128), (100, 264, 1536), (260, 2600, 4160)])
@@ -611,17 +624,32 @@ def test_swiglu_rows_of_unlike_gate_and_up(rows, n, k):
 
 @pytest.mark.parametrize(
     ("rows", "n", "k"),
-    [(65, 72, 64),        # one group: two steps; the second half holds one row
-     (128, 130, 192),     # a full tile
-     (129, 300, 320),     # the last tile's second half empty
-     (200, 264, 4160),    # 65 groups in K ranges of whole groups
-     (333, 1536, 8960),   # the module path's down projection
-     (600, 28000, 192)],  # more tiles than workgroup slots: whole and split ones
+    [(2049, 130, 64),      # one group; the last tile one row of 128 and two columns of 256; eight waves
+     (2113, 300, 320),     # one row in the last tile's second half
+     (2177, 77, 704),      # odd feature count; K ranges of 3 groups (two planes: of 4 steps), the last one shorter
+     (2100, 264, 4160),    # 65 groups; two planes: ranges of 19 steps made 20
+     (2049, 7930, 1024),   # 512 whole tiles and 15 in K ranges
+     (513, 17000, 320)],   # unsplit tiles of four waves, two workgroups per CU
+)
+@pytest.mark.parametrize("dtype", ["fp16", "bf16", "fp32"])
+def test_tiles_at_their_edges(rows, n, k, dtype):
+    """The 128 x 256 tiles with ragged rows, features and groups."""
+    check_exact_products(rows, n, k, dtype, "128x256")
+
+
+@pytest.mark.parametrize(
+    ("rows", "n", "k"),
+    [(1025, 72, 64),       # one group: two steps; the last tile holds one row
+     (1089, 300, 320),     # one row in the last tile's second half; K ranges of one group
+     (1152, 130, 192),     # full tiles
+     (333, 1536, 8960),    # the module path's down projection
+     (1025, 14500, 192),   # 512 whole tiles and one in K ranges of one step made two
+     (600, 28000, 192)],   # more tiles than workgroup slots, all whole
 )
 def test_two_planes_in_one_sum(rows, n, k):
     """fp32 rows of the 128 x 256 tiles: both planes of a group in one sum, at
-    the edges of the row halves, K ranges and tiles (bound as above)."""
-    test_few_row_tiles(rows, n, k, "fp32")
+    the edges of the row halves, K ranges and tiles."""
+    check_exact_products(rows, n, k, "fp32", "128x256")
 
 
 @pytest.mark.parametrize(
@@ -630,12 +658,16 @@ def test_two_planes_in_one_sum(rows, n, k):
      (200, 1300, 320),   # blocks of four, eight waves
      (300, 4112, 1024),  # more than one workgroup per CU: four waves
      (333, 40, 10304),   # 161 groups: two K ranges over row blocks
+     (65, 72, 64),
+     (128, 130, 192),
+     (129, 300, 320),
+     (200, 264, 4160),   # 65 groups
      (1024, 48, 64),     # many row blocks of one group
      (2048, 33, 192)],   # the most rows (two planes: the tiled kernel)
 )
 @pytest.mark.parametrize("dtype", ["fp16", "bf16", "fp32"])
 def test_row_blocks(rows, n, k, dtype):
-    test_few_row_tiles(rows, n, k, dtype)
+    check_exact_products(rows, n, k, dtype, "128x256" if dtype == "fp32" and rows > 1024 else "few rows")
 
 
 @pytest.mark.parametrize("rows,n,k,dtype", [
@@ -663,9 +695,9 @@ def test_gemm_is_chosen_by_the_problem_alone(rows, n, k, dtype):
     assert torch.equal(*got)
 
 
-@pytest.mark.parametrize("rows,n,k", [(70, 72, 64), (160, 520, 1984), (260, 2600, 4160)])
+@pytest.mark.parametrize("rows,n,k", [(1025, 72, 64), (1100, 520, 1984), (260, 2600, 4160)])
 def test_two_planes_of_the_swiglu_product(rows, n, k):
-    test_few_row_tiles_of_the_swiglu_product(rows, n, k)
+    check_swiglu_products(rows, n, k, "128x256")
 
 
 @pytest.mark.parametrize(
