@@ -16,15 +16,14 @@
 //                       probability-weighted value sums.  The last workgroup
 //                       of a (sequence, head) to arrive merges the chunks
 //                       (rescaled by exp(m_chunk - m)) and writes bf16
-//                       (model.py:61-122).  Batch 1 and up to 16 chunks;
-//                       larger calls take qwen2_decode_split.hip.
-//   prefill_rope_kernel, prefill_attention_kernel
-//                       a prompt: rotary of every position (queries to a
-//                       workspace, keys and values into the caches), then
-//                       causal GQA attention, one workgroup per (sequence,
-//                       head, 64 query rows) over 64-key blocks staged in LDS,
-//                       online softmax (model.py:17-31, :61-122).
+//                       (model.py:61-122).  Up to 16 chunks: one sequence,
+//                       or batches of up to 96 chunks in all whose context
+//                       the split kernel would divide; other calls take
+//                       qwen2_decode_split.hip.
 //   silu_mul_kernel     silu(gate) * up in fp32 (model.py:133-136).
+//
+// The entry points of a prompt's attention are here, their kernels in
+// qwen2_prefill.hip.
 //
 // The new key at position p is read by the chunk that holds p from LDS, never
 // from the cache, so no workgroup reads a cache row another one is writing.

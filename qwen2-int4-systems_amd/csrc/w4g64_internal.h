@@ -214,8 +214,8 @@ hipError_t launch_gemm(const LinearProblem& p, void* workspace, int64_t workspac
 // The allocation-free entry point's scratch (w4g64_linear_static_scratch).
 constexpr int64_t kScratchBytes = 4ll << 20;
 
-// GEMM of a few row tiles (w4g64_gemm_rows.hip): 17 to 128 rows, fp32-class
-// kinds to 64.  Workspace: [split-K partial sums][staged rows][row factors].
+// GEMM of few products (w4g64_gemm_rows.hip): 17 rows up to 2048, fp32-class
+// kinds to 1024, where plan_rows says so.  Workspace: [split-K partial sums][staged rows][row factors].
 struct RowsPlan {
     bool taken;  // false: the prefill GEMM
     int tiles;   // 16-row tiles per row block, 2 to 4

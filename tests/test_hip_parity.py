@@ -346,8 +346,8 @@ def test_fp32_activations_run_natively(rows):
     q, s, z = weights("sym", n, k, O.BASE_SEED + n + k)
     x = O.activations(rows, k, seed=O.BASE_SEED + 5 * rows, dtype="fp32")
     bias = np.linspace(-1, 1, n, dtype=np.float32)
-    # decode splits fp32 exactly into three bf16 parts; the GEMM into two
-    # (|x - hi - lo| <= 2^-17 |x|) against exact weights: near-fp32 accuracy
+    # decode splits fp32 exactly into three bf16 parts; the GEMM into two of fp16
+    # (|x - hi - lo| <= 2^-22 |x|) against exact weights: near-fp32 accuracy
     check_linear(x, q, s, z, bias, n, k, "fp32", bias_dtype="fp32", normwise=1e-5, tol=(1e-4, 1e-4))
 
 
