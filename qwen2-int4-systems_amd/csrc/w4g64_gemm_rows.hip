@@ -26,7 +26,7 @@
 // graph-replayed over rotated weights, against the 128 x 256 tiles: 24 x
 // 17920x1536 29.0 -> 11.6 us, 24 x 1536x1536 16.0 -> 6.8, 40 x 8960x1536 23.1
 // -> 11.1, 128 x 8960x1536 27.9 -> 16.1, 512 x 1536x1536 24.7 -> 14.3, 24 x
-// 1536x8960 of the SwiGLU product (fp32) 33.2 -> 16.6, 64 x 1536x8960 fp32 32.7
+// 1536x8960 of the SwiGLU product (fp32) 33.2 -> 17.1, 64 x 1536x8960 fp32 32.7
 // -> 22.4.
 #include "w4g64_gemm.h"
 #include "w4g64_internal.h"
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(THREADS) void rows_stage_kernel(const void* x, u32x
     }
 }
 
-// The SwiGLU product, one workgroup per row and 2048 values: its exponentials
+// The SwiGLU product, one workgroup per row and 4096 values: its exponentials
 // and divisions, on one CU per row, took 7.0 us at 24 x 8960.  Every
 // workgroup of a row scans all of it for the largest finite product, so they
 // agree on the row's factor.  The scan's products come of the exponential and
@@ -139,14 +139,17 @@ __global__ __launch_bounds__(THREADS) void rows_stage_kernel(const void* x, u32x
 // factor of a row whose maximum lies that close to a power of two, and the
 // largest staged value from [2^14, 2^15) to at most 2^15 (1 + 2^-16).
 // (max|gate| times max|up| in its place loses the row where they lie in
-// different columns or the gate is negative; the products cost 0.3 us of a
-// call of 24 x 1536x8960, 16.3 -> 16.6, and 0.4 of 64 rows, 24.0 -> 24.5.)
-__global__ __launch_bounds__(256) void rows_stage_swiglu_kernel(const void* x, u32x4* out, float* rowscale, int K) {
-    __shared__ float wmax[4];
+// different columns or the gate is negative.)  Threads per workgroup, us per
+// call of 24, 64 and 160 x 1536x8960: 256 17.05, 25.0, 31.4; 512 17.1, 24.0,
+// 30.5; 1024 18.3, 25.5, 31.3 (16.7, 24.4, 30.1 were those of the lost rows).
+constexpr int kSwigluThreads = 512;
+__global__ __launch_bounds__(kSwigluThreads) void rows_stage_swiglu_kernel(const void* x, u32x4* out, float* rowscale,
+                                                                          int K) {
+    __shared__ float wmax[kSwigluThreads / 64];
     const int m = blockIdx.x;
     const int chunks = K / 8;
     const uint16_t* gu = (const uint16_t*)x + (int64_t)m * 2 * K;
-    const int own = blockIdx.y * 256 + threadIdx.x;
+    const int own = blockIdx.y * kSwigluThreads + threadIdx.x;
     float v[8];
     if (own < chunks) stage_load8<kSwiGLU>(x, m, K, own, v);
     float mx = 0.0f;
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(256) void rows_stage_swiglu_kernel(const void* x, u
         const float p = (fabsf(g) * 0x1p-8f) * __builtin_amdgcn_rcpf(__builtin_fmaf(e, 0x1p-8f, 0x1p-8f)) * fabsf(u);
         mx = p < INFINITY ? fmaxf(mx, p) : mx;  // (neither infinite nor NaN)
     };
-    for (int c = threadIdx.x; c < chunks; c += 256) {
+    for (int c = threadIdx.x; c < chunks; c += kSwigluThreads) {
         const u32x4 g = *(const u32x4*)(gu + 8 * c), u = *(const u32x4*)(gu + K + 8 * c);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -169,8 +172,10 @@ __global__ __launch_bounds__(256) void rows_stage_swiglu_kernel(const void* x, u
     mx = wave_max64(mx);
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
     __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kSwigluThreads / 64; ++w) mx = fmaxf(mx, wmax[w]);
     float inv, rs;
-    row_factors(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])), inv, rs);
+    row_factors(mx, inv, rs);
     if (threadIdx.x == 0 && blockIdx.y == 0) rowscale[m] = rs;
     if (own < chunks) {
         u32x4 hi, lo;
@@ -516,8 +521,9 @@ hipError_t launch_rows(const LinearProblem& p, const RowsPlan& pl, void* workspa
         case kF16: err = launch_stage<kF16>(p, staged, rowscale, stream, start); break;
         case kBF16: err = launch_stage<kBF16>(p, staged, rowscale, stream, start); break;
         case kSwiGLU:
-            err = launch_kernel(rows_stage_swiglu_kernel, dim3((unsigned)p.rows, (unsigned)((p.in_features / 8 + 255) / 256)),
-                                dim3(256), 0, stream, start, nullptr, p.x, staged, rowscale, (int)p.in_features);
+            err = launch_kernel(rows_stage_swiglu_kernel,
+                                dim3((unsigned)p.rows, (unsigned)((p.in_features / 8 + kSwigluThreads - 1) / kSwigluThreads)),
+                                dim3(kSwigluThreads), 0, stream, start, nullptr, p.x, staged, rowscale, (int)p.in_features);
             break;
         default: err = launch_stage<kF32>(p, staged, rowscale, stream, start); break;
     }
