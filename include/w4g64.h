@@ -91,8 +91,9 @@ int w4g64_dequantize_canonical(const uint8_t* qweight, const uint16_t* scales, c
 /* Bytes of workspace w4g64_linear needs for this problem (0 = none).
  * It holds fp32 split-K partial sums (decode shapes that split K across
  * workgroups; prefill shapes whose tiles do not fill whole rounds of the
- * device's workgroup slots, up to 64 MiB) -- and, for fp32 activations of the
- * prefill GEMM, their two bf16 planes.  Every call writes what it reads, so a
+ * device's workgroup slots, up to 64 MiB) -- and, past 16 rows, the activation
+ * rows staged as fp16 (two planes for fp32 ones).  A larger workspace changes
+ * nothing about the kernel that runs.  Every call writes what it reads, so a
  * workspace needs no initial contents: a caller allocates one (sized for its
  * largest problem) and reuses it for every shape.  Calls sharing a workspace
  * must be ordered on one stream.  The prefill plan depends on the current
@@ -159,7 +160,7 @@ int w4g64_stream_probe(const void* src, int64_t bytes, void* sink, void* stream)
  * h = silu(gate) * up in fp32 (silu(g) = g / (1 + exp(-g))), and
  * y[rows, out] = h @ dequant(W)^T (+ bias) in fp32, as w4g64_linear on the
  * fp32 h (decode rows 1..16: formed in the GEMV's activation staging; more
- * rows: written as the GEMM's bf16 planes).  gate_up and qweight 16-byte
+ * rows: staged as the GEMM's two fp16 planes).  gate_up and qweight 16-byte
  * aligned.
  * Replaces: QwenMLP.forward's product and down projection
  *           (src/qwen_int4/model.py:133-136). */
