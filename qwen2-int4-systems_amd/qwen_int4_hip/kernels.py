@@ -275,10 +275,14 @@ def cached_attention_hip(q, k, v, cos, sin, past, mask, *, num_heads: int, num_k
             or mask.device != device or not batch * length
             or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors))):
         return None
-    length_past = 0 if past is None or past[0].ndim != 4 else past[0].shape[2]
+    length_past = 0
+    if past is not None:
+        kept = past[0].shape
+        length_past = kept[2] if len(kept) == 4 else 0
+        if len(past) != 2 or kept != (batch, num_kv_heads, length_past, 128) or past[1].shape != kept:
+            return None
     total = length_past + length
-    if (tuple(mask.shape) != (batch, total)
-            or past is not None and [tuple(t.shape) for t in past] != 2 * [(batch, num_kv_heads, length_past, 128)]):
+    if mask.shape != (batch, total):
         return None
     # (contiguous and aligned already where the linears and this function made them)
     q, k, v, cos, sin = (t.contiguous() for t in (q, k, v, cos, sin))
@@ -288,7 +292,7 @@ def cached_attention_hip(q, k, v, cos, sin, past, mask, *, num_heads: int, num_k
     new_k = torch.empty((batch, num_kv_heads, total, 128), dtype=torch.bfloat16, device=device)
     new_v = torch.empty_like(new_k)
     out = torch.empty((batch, length, num_heads * 128), dtype=torch.bfloat16, device=device)
-    lib = _require_library()
+    lib = _lib.load()
     _lib.check(lib.qwen2_cached_attention(
         *map(_ptr, (q, k, v, cos, sin, past_k, past_v, mask, new_k, new_v, out)), batch, length, length_past, num_heads,
         num_kv_heads, 128, ctypes.c_float(128 ** -0.5), _stream_handle(device)))

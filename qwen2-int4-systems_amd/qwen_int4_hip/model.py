@@ -115,9 +115,9 @@ class QwenAttention(nn.Module):
     def _fused(self, attention_mask) -> bool:
         """Whether the layer may take the HIP attention: every projection on the
         HIP backend (the others are its references), heads of 128, a key mask
-        (``QwenModel`` always passes one).  What the tensors themselves rule
-        out, ``cached_attention_hip`` answers."""
-        return (self.head_dim == 128 and attention_mask is not None and torch.cuda.is_available()
+        (``QwenModel`` always passes one) on a GPU.  What the tensors themselves
+        rule out, ``cached_attention_hip`` answers."""
+        return (self.head_dim == 128 and attention_mask is not None and attention_mask.is_cuda
                 and all(getattr(p, "backend", None) == "hip"
                         for p in (self.q_proj, self.k_proj, self.v_proj, self.o_proj)))
 

@@ -288,7 +288,7 @@ def test_full_workload_fused_serving_path_against_reference_backend():
     assert torch.equal(picked[clear], ref_tokens[clear])
 
 
-def test_attention_layer_takes_projections_of_another_kind(monkeypatch):
+def test_attention_layer_takes_projections_of_another_kind():
     """A projection replaced by any other module (here ``nn.Linear``) runs."""
     from qwen_int4_hip import PackingFormat
     from qwen_int4_hip.model import QwenAttention
@@ -300,6 +300,5 @@ def test_attention_layer_takes_projections_of_another_kind(monkeypatch):
         setattr(layer, name, torch.nn.Linear(proj.in_features, proj.out_features, dtype=torch.bfloat16))
     hidden, factors = torch.randn(1, 3, 256).bfloat16(), torch.ones(1, 3, 128).bfloat16()
     with torch.no_grad():
-        want = layer(hidden, factors, factors, torch.ones(1, 3))[0]
-        monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
-        assert torch.equal(layer(hidden, factors, factors, torch.ones(1, 3))[0], want)
+        assert layer(hidden, factors, factors, torch.ones(1, 3))[0].shape == hidden.shape
+    assert not layer._fused(SimpleNamespace(is_cuda=True))  # (a mask on a GPU)
