@@ -14,6 +14,7 @@ import ctypes
 import threading
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -242,8 +243,11 @@ def linear_kernel_name(rows: int, out_features: int, in_features: int, dtype: to
 def _operators_followed() -> bool:
     """Whether a function or dispatch mode, ``torch.jit.trace``, a functorch
     level, forward-mode differentiation or ``torch.compile`` follows torch's
-    operators, which see nothing of a call into the library."""
-    return (torch.compiler.is_compiling() or torch._C._len_torch_function_stack() > 0
+    operators, which see nothing of a call into the library.  (A default device
+    is a function mode too, but only for the functions that make tensors.)"""
+    return (torch.compiler.is_compiling()
+            or any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+                   for i in range(torch._C._len_torch_function_stack()))
             or torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0)

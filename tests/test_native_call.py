@@ -128,8 +128,10 @@ def test_what_follows_torch_operators_is_seen():
     from torch.utils._python_dispatch import TorchDispatchMode
 
     assert not kernels._operators_followed()
+    with torch.device("cpu"):  # (a default device is no such state)
+        assert not kernels._operators_followed()
     for mode in (TorchFunctionMode(), TorchDispatchMode(), forward_ad.dual_level()):
-        with mode:
+        with torch.device("cpu"), mode:
             assert kernels._operators_followed(), type(mode)
     seen = []
     torch.func.vmap(lambda t: (seen.append(kernels._operators_followed()), t)[1])(torch.zeros(2))
